@@ -456,8 +456,9 @@ __device__ __forceinline__ void compute_pairs(const Stage<D, BF16, FP8> (&st)[NP
 // The same wave reads the page back later in program order (its own store
 // to the same addresses comes first), so the attention sees the new row
 // exactly as the pool holds it, with no patching of loaded registers.
-// With ROPE the K row is rotated first (position `pos`): lane c < D/16 takes
-// the chunk pair c, c + D/16 (elements i and i + D/2).
+// With ROPE the K row is rotated first, by the row's position, whose
+// rope_table the caller has made in rope_tab: lane c < D/16 takes the chunk
+// pair c, c + D/16 (elements i and i + D/2).
 template <int D, bool BF16, bool FP8>
 __device__ __forceinline__ void put_chunk(const DecodeParams& p, int h, int page, int slot,
                                           int is_v, int c, u32x4 x) {
@@ -479,7 +480,8 @@ __device__ __forceinline__ void put_chunk(const DecodeParams& p, int h, int page
 
 template <int D, bool BF16, bool FP8, bool ROPE>
 __device__ __forceinline__ void fused_append(const DecodeParams& p, int b, int h,
-                                             int page, int slot, int lane, int pos) {
+                                             int page, int slot, int lane,
+                                             const float* rope_tab) {
   const int is_v = lane >> 5;
   const int c = lane & 31;
   if (c >= D / 8) return;
@@ -491,9 +493,7 @@ __device__ __forceinline__ void fused_append(const DecodeParams& p, int b, int h
     u32x4 lo = *reinterpret_cast<const u32x4*>(src + 8 * c);
     u32x4 hi = *reinterpret_cast<const u32x4*>(src + 8 * c + D / 2);
     float cs[8], sn[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      rope_cos_sin(pos, 8 * c + e, D, p.rope_inv_scale, p.rope_log2_theta, &cs[e], &sn[e]);
+    rope_table8<D>(rope_tab, 8 * c, cs, sn);
     rope8<BF16>(lo, hi, cs, sn);
     put_chunk<D, BF16, FP8>(p, h, page, slot, 0, c, lo);
     put_chunk<D, BF16, FP8>(p, h, page, slot, 0, c + D / 16, hi);
@@ -567,6 +567,8 @@ __global__ void __launch_bounds__(256, 1) decode_kernel(DecodeParams p) {
   const int n = lane & 15;
   const int G = lane >> 4;
   const int g = p.g;
+  __shared__ __attribute__((aligned(16))) float rope_tabs[ROPE ? 4 : 1][ROPE ? D : 4];
+  float* rope_tab = rope_tabs[ROPE ? wave : 0];
 
   // one work item: pages [item_lo, item_hi) of sequence b for KV heads
   // h0 + [0, hg); slot0 >= 0: the item is one piece of a cut sequence and
@@ -599,15 +601,12 @@ __global__ void __launch_bounds__(256, 1) decode_kernel(DecodeParams p) {
       if (p.new_pos) new_pos = uniform(load_invariant(p.new_pos + b));
     }
     if constexpr (ROPE) {
-      const int rope_at = new_pos;
+      rope_table<D>(rope_tab, new_pos, p.rope_inv_scale, p.rope_log2_theta, lane);
       // d and d + D/2 sit in the same lane: fragments ks and ks + D/64
 #pragma unroll
       for (int ks = 0; ks < D / 64; ++ks) {
         float cs[8], sn[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          rope_cos_sin(rope_at, 32 * ks + 8 * G + e, D, p.rope_inv_scale,
-                       p.rope_log2_theta, &cs[e], &sn[e]);
+        rope_table8<D>(rope_tab, 32 * ks + 8 * G, cs, sn);
         rope8<BF16>(qf[ks], qf[ks + D / 64], cs, sn);
       }
     }
@@ -623,7 +622,7 @@ __global__ void __launch_bounds__(256, 1) decode_kernel(DecodeParams p) {
         if (pg >= page_lo && pg < page_hi) {
           const int page = page_id(p, ind_lo, pg, npages);
           if (page >= 0) {
-            fused_append<D, BF16, FP8, ROPE>(p, b, h, page, new_slot, lane, new_pos);
+            fused_append<D, BF16, FP8, ROPE>(p, b, h, page, new_slot, lane, rope_tab);
           } else {
             skipped = true;
           }
@@ -781,6 +780,7 @@ struct SharedLds {
       n_chunks[kSharedMaxItems], ind_lo[kSharedMaxItems], npages[kSharedMaxItems],
       last[kSharedMaxItems], new_pos[kSharedMaxItems];
   u32x4 q[kSharedMaxItems][D / 32][kWave];  // Q B-operands (rotated with ROPE)
+  float rope[4][D];  // per wave: cosines and sines of one position (rope_table)
   struct State {
     f32x4 o[D / 16][kWave];
     float m[kWave], l[kWave];
@@ -1122,14 +1122,11 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
       const int i = wave + 4 * k;
       if (i < n_it) {
         if constexpr (ROPE) {
-          const int rope_at = field(t_pos, i);
+          rope_table<D>(L.rope[wave], field(t_pos, i), p.rope_inv_scale, p.rope_log2_theta, lane);
 #pragma unroll
           for (int ks = 0; ks < D / 64; ++ks) {
             float cs[8], sn[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              rope_cos_sin(rope_at, 32 * ks + 8 * G + e, D, p.rope_inv_scale,
-                           p.rope_log2_theta, &cs[e], &sn[e]);
+            rope_table8<D>(L.rope[wave], 32 * ks + 8 * G, cs, sn);
             rope8<BF16>(qtmp[k][ks], qtmp[k][ks + D / 64], cs, sn);
           }
         }
@@ -1157,10 +1154,13 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
     const int pg = pos >= 0 ? pos / kPage : -1;
     if (b < 0 || pg < 0 || pg >= np) return;
     const int page = page_id(p, field(t_ind, i), pg, np);
-    if (page >= 0)
-      fused_append<D, BF16, FP8, ROPE>(p, b, h, page, pos & (kPage - 1), lane, pos);
-    else
+    if (page >= 0) {
+      if constexpr (ROPE)
+        rope_table<D>(L.rope[wave], pos, p.rope_inv_scale, p.rope_log2_theta, lane);
+      fused_append<D, BF16, FP8, ROPE>(p, b, h, page, pos & (kPage - 1), lane, L.rope[wave]);
+    } else {
       count_lanes(p.append_err, h == 0 && lane == 0);
+    }
   };
   if constexpr (APPEND) {
     if (det) {
