@@ -1,6 +1,7 @@
 // Small kernels of the path: batch index / position expansion, RoPE, page
 // append (bf16/fp16 copy or e4m3 quantise), fp8 pool builder, HBM copy.
 // All are HBM- or latency-bound; none reads a byte twice.
+#include <algorithm>
 #include <cmath>
 
 #include "append.h"
@@ -112,70 +113,122 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
 // ----------------------------------------------------------------------------
 // RoPE + append in one launch: what apply_rope_pos_ids_inplace
 // (src/models/llama.py:175-182, non-interleaved, full head) followed by
-// append_paged_kv_cache (:188-210) do.  Threads [0, nnz * D/16) own (token,
-// frequency chunk of 8): sin/cos once, then every q head rotated in place and
-// every k head rotated in place and written to its page slot.  The remaining
-// threads copy the V rows, one 16-byte chunk each.
+// append_paged_kv_cache (:188-210) do.  Memory- and latency-bound.  A
+// workgroup owns T tokens (grid y: one block of kRopeFreqs frequencies, a
+// single one up to head_dim 128).  A token's units are its hq q heads, hkv k
+// heads and hkv v heads; 8 lanes (fewer where the head has fewer chunk pairs)
+// work a unit, lane c the 16-byte chunk c of the head's first half and its
+// partner half a head away.  Wave w evaluates token w's cosines and sines, one
+// frequency per lane, into LDS, and the last wave looks the tokens' pages up,
+// while every thread's first rows are already on their way.
+//
+// Before, one thread owned (token, 8 frequencies) and walked all heads one
+// after the other: a 512-token step of a 32/8-head layer kept 16 of 256 CUs
+// busy for 19.9 us.
 struct RopeAppendArgs {
   AppendArgs a;
   uint16_t* q;
   int64_t q_sn, q_sh;
   int32_t hq;
+  int32_t tokens;   // T, 1 to kRopeMaxTokens
+  int32_t c_shift;  // log2 of the lanes per unit
   double inv_scale, log2_theta;
 };
 
+constexpr int kRopeFreqs = 64;
+constexpr int kRopeMaxTokens = 4;  // one wave's table each
+constexpr int kRopeBatch = 4;      // units a thread has in flight
+
 template <bool IS_BF16, bool TO_FP8>
 __global__ void __launch_bounds__(256) rope_append_kernel(RopeAppendArgs r) {
+  __shared__ __attribute__((aligned(16))) float tab[kRopeMaxTokens][2][kRopeFreqs];
+  __shared__ int64_t pages[kRopeMaxTokens];
+  __shared__ int slots[kRopeMaxTokens];
   const AppendArgs& a = r.a;
   const int d = a.d;
-  const int nrot = d >> 4;  // frequency chunks of 8 per token
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n_rot = (int64_t)a.nnz * nrot;
-  if (t < n_rot) {
-    const int j = (int)(t / nrot);
-    const int c = (int)(t % nrot);
-    float cs[8], sn[8];
-    const int pos = a.positions[j];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = uniform(threadIdx.x >> 6);
+  const int f0 = (int)blockIdx.y * kRopeFreqs;        // first frequency of this block
+  const int npair = min(kRopeFreqs, d / 2 - f0) / 8;  // chunk pairs of a head here
+  const int64_t j0 = (int64_t)blockIdx.x * r.tokens;
+  const int nt = (int)min<int64_t>(r.tokens, a.nnz - j0);
+  const int per_tok = r.hq + 2 * a.hkv;
+  const int n_units = nt * per_tok;
+  const int c = threadIdx.x & ((1 << r.c_shift) - 1);
+  const int step = 256 >> r.c_shift;
+  const int e0 = f0 + 8 * c;  // element of the lane's first chunk
+
+  // unit u of the workgroup: its row, and h < hq: q head h, then k and v heads
+  auto row_of = [&](int u, int* tok, int* h) -> uint16_t* {
+    const int t = u / per_tok;
+    const int x = u - t * per_tok;
+    const int64_t j = j0 + t;
+    *tok = t;
+    *h = x;
+    if (x < r.hq) return r.q + j * r.q_sn + (int64_t)x * r.q_sh;
+    if (x < r.hq + a.hkv)
+      return const_cast<uint16_t*>(a.k) + j * a.k_sn + (int64_t)(x - r.hq) * a.k_sh;
+    return const_cast<uint16_t*>(a.v) + j * a.v_sn + (int64_t)(x - r.hq - a.hkv) * a.v_sh;
+  };
+  u32x4 lo[kRopeBatch], hi[kRopeBatch];
+  auto load = [&](int u0) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      rope_cos_sin(pos, 8 * c + e, d, r.inv_scale, r.log2_theta, &cs[e], &sn[e]);
-    for (int h = 0; h < r.hq; ++h) {
-      uint16_t* x = r.q + (int64_t)j * r.q_sn + (int64_t)h * r.q_sh;
-      u32x4 lo = *reinterpret_cast<const u32x4*>(x + 8 * c);
-      u32x4 hi = *reinterpret_cast<const u32x4*>(x + 8 * c + d / 2);
-      rope8<IS_BF16>(lo, hi, cs, sn);
-      *reinterpret_cast<u32x4*>(x + 8 * c) = lo;
-      *reinterpret_cast<u32x4*>(x + 8 * c + d / 2) = hi;
-    }
-    int slot = 0;
-    const int64_t page = append_target_page(a, j, &slot);
-    count_lanes(a.err, page < 0 && c == 0);
-    for (int h = 0; h < a.hkv; ++h) {
-      uint16_t* x = const_cast<uint16_t*>(a.k) + (int64_t)j * a.k_sn + (int64_t)h * a.k_sh;
-      u32x4 lo = *reinterpret_cast<const u32x4*>(x + 8 * c);
-      u32x4 hi = *reinterpret_cast<const u32x4*>(x + 8 * c + d / 2);
-      rope8<IS_BF16>(lo, hi, cs, sn);
-      *reinterpret_cast<u32x4*>(x + 8 * c) = lo;
-      *reinterpret_cast<u32x4*>(x + 8 * c + d / 2) = hi;
-      if (page >= 0) {
-        store_chunk<IS_BF16, TO_FP8>(a, page, slot, 0, h, 8 * c, lo);
-        store_chunk<IS_BF16, TO_FP8>(a, page, slot, 0, h, 8 * c + d / 2, hi);
+    for (int k = 0; k < kRopeBatch; ++k) {
+      const int u = u0 + k * step;
+      if (u < n_units && c < npair) {
+        int tok, h;
+        const uint16_t* x = row_of(u, &tok, &h);
+        lo[k] = *reinterpret_cast<const u32x4*>(x + e0);
+        hi[k] = *reinterpret_cast<const u32x4*>(x + e0 + d / 2);
       }
     }
-    return;
+  };
+  int u0 = threadIdx.x >> r.c_shift;
+  load(u0);
+  if (wave < nt && lane < 8 * npair) {
+    float cs, sn;
+    rope_cos_sin(a.positions[j0 + wave], f0 + lane, d, r.inv_scale, r.log2_theta, &cs, &sn);
+    tab[wave][0][lane] = cs;
+    tab[wave][1][lane] = sn;
   }
-  const int chunks = d >> 3;
-  const int64_t u = t - n_rot;
-  if (u >= (int64_t)a.nnz * a.hkv * chunks) return;
-  const int c = (int)(u % chunks);
-  const int h = (int)((u / chunks) % a.hkv);
-  const int j = (int)(u / ((int64_t)chunks * a.hkv));
-  int slot = 0;
-  const int64_t page = append_target_page(a, j, &slot);
-  if (page < 0) return;
-  const u32x4 x = *reinterpret_cast<const u32x4*>(a.v + (int64_t)j * a.v_sn +
-                                                  (int64_t)h * a.v_sh + 8 * c);
-  store_chunk<IS_BF16, TO_FP8>(a, page, slot, 1, h, 8 * c, x);
+  if (wave == 256 / kWave - 1 && lane < nt) {
+    int slot = 0;
+    const int64_t page = append_target_page(a, (int)j0 + lane, &slot);
+    pages[lane] = page;
+    slots[lane] = slot;
+    count_lanes(a.err, page < 0 && blockIdx.y == 0);
+  }
+  __syncthreads();
+  while (true) {
+#pragma unroll
+    for (int k = 0; k < kRopeBatch; ++k) {
+      const int u = u0 + k * step;
+      if (u >= n_units || c >= npair) continue;
+      int tok, h;
+      uint16_t* x = row_of(u, &tok, &h);
+      if (h < r.hq + a.hkv) {
+        float cs[8], sn[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          cs[e] = tab[tok][0][8 * c + e];
+          sn[e] = tab[tok][1][8 * c + e];
+        }
+        rope8<IS_BF16>(lo[k], hi[k], cs, sn);
+        *reinterpret_cast<u32x4*>(x + e0) = lo[k];
+        *reinterpret_cast<u32x4*>(x + e0 + d / 2) = hi[k];
+        if (h < r.hq) continue;
+      }
+      const int64_t page = pages[tok];
+      if (page < 0) continue;
+      const int kind = h >= r.hq + a.hkv ? 1 : 0;
+      const int kvh = h - r.hq - kind * a.hkv;
+      store_chunk<IS_BF16, TO_FP8>(a, page, slots[tok], kind, kvh, e0, lo[k]);
+      store_chunk<IS_BF16, TO_FP8>(a, page, slots[tok], kind, kvh, e0 + d / 2, hi[k]);
+    }
+    u0 += kRopeBatch * step;
+    if (u0 >= n_units) break;
+    load(u0);
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -474,9 +527,18 @@ int pagedattn_rope_append_paged_kv_cache(
   r.hq = num_qo_heads;
   r.inv_scale = 1.0 / (double)rope_scale;
   r.log2_theta = std::log2((double)rope_theta);
-  const int64_t threads = (int64_t)nnz * (head_dim / 16) +
-                          (int64_t)nnz * num_kv_heads * (head_dim / 8);
-  const dim3 grid((unsigned)((threads + 255) / 256));
+  // lanes per unit: the chunk pairs of a head (a block's 8 at most), rounded
+  // up to a power of two
+  const int pairs = std::min(head_dim / 16, kRopeFreqs / 8);
+  r.c_shift = 0;
+  while ((1 << r.c_shift) < pairs) ++r.c_shift;
+  // tokens per workgroup: as many as one batch of loads covers (a token of few
+  // heads does not fill 256 threads by itself)
+  const int64_t lanes = ((int64_t)num_qo_heads + 2 * (int64_t)num_kv_heads) << r.c_shift;
+  r.tokens = (int)std::min<int64_t>(kRopeMaxTokens,
+                                    std::max<int64_t>(1, 256 * kRopeBatch / 2 / lanes));
+  const dim3 grid((unsigned)(((int64_t)nnz + r.tokens - 1) / r.tokens),
+                  (unsigned)((head_dim / 2 + kRopeFreqs - 1) / kRopeFreqs));
   hipStream_t s = (hipStream_t)stream;
   const bool bf16 = src_dtype == PAGEDATTN_BF16;
   if (cache_dtype != PAGEDATTN_E4M3) {

@@ -247,3 +247,40 @@ def test_rope_append_equals_separate(gpu, dtype, prefill, fp8):
         clamped = O.e4m3_clamped_pieces(k_a.cpu().float(), v.cpu().float(), scales.cpu(), bi,
                                         pos, meta.kv_indices, meta.kv_indptr, pool.shape[0])
     assert err_a.tolist() == err_b.tolist() == [1, clamped]
+
+
+@pytest.mark.parametrize("d,hq,hkv,nnz", [
+    (16, 1, 1, 1),      # one chunk pair a head, one token
+    (48, 3, 1, 7),      # pairs not a power of two, tokens not a multiple of the workgroup's
+    (64, 32, 4, 33),
+    (128, 8, 1, 5),     # few heads: four tokens a workgroup
+    (128, 64, 8, 18),   # more units than one batch of loads
+    (160, 2, 2, 9),     # two frequency blocks, the second partial
+    (256, 16, 16, 3),
+])
+def test_rope_append_shapes_equal_separate(gpu, d, hq, hkv, nnz):
+    # the workgroup split of the fused launch at its edges: same bits as the
+    # two calls, for every head of q, k and v and every page slot
+    g = torch.Generator(device=gpu)
+    g.manual_seed(d + hq)
+    n_pages = -(-nnz // 16) + 1
+    pool = torch.randn((n_pages, 2, hkv, 16, d), generator=g, device=gpu).to(torch.bfloat16)
+    qkv = torch.randn((nnz, (hq + 2 * hkv) * d), generator=g, device=gpu).to(torch.bfloat16)
+    ind = i32(np.arange(n_pages)[::-1].copy(), gpu)
+    indptr, last = i32([0, n_pages], gpu), i32([nnz % 16 + 1], gpu)
+    bi, pos = i32(np.zeros(nnz), gpu), i32(np.arange(1, nnz + 1), gpu)
+
+    def views(x):
+        q, k, v = x.split([hq * d, hkv * d, hkv * d], dim=-1)
+        return q.view(nnz, hq, d), k.view(nnz, hkv, d), v.view(nnz, hkv, d)
+
+    a, b, pool_a, pool_b = qkv.clone(), qkv.clone(), pool.clone(), pool.clone()
+    q, k, v = views(a)
+    pagedattn.apply_rope_pos_ids_inplace(q, k, pos, rope_theta=500000.0)
+    pagedattn.append_paged_kv_cache(k, v, bi, pos, pool_a, ind, indptr, last, kv_layout="HND")
+    q, k, v = views(b)
+    pagedattn.rope_append_paged_kv_cache(q, k, v, bi, pos, pool_b, ind, indptr, last,
+                                         kv_layout="HND", rope_theta=500000.0)
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+    assert torch.equal(pool_a, pool_b)
