@@ -1303,44 +1303,120 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
 
 // Combine the base-2 partials of n pieces, slot_of(s) giving piece s's
 // (slot * g + head) index: M = max lse, den = sum 2^(lse - M), num = sum
-// 2^(lse - M) o[dd].  The lse and o of up to four pieces are loaded together,
-// so the o loads do not wait for the max; later batches rescale the sums.
-template <typename SlotOf>
+// 2^(lse - M) o, out = num / den.  Pieces s, s + 8, s + 16, ... form class
+// s mod 8; a wave sums a class, kMergeBatch loads at a time, and the classes
+// are added in order, so the bits depend on the piece count alone and not on
+// the workgroup's waves (any number from D / 64 to 8).
+//
+// Bound by the latency of dependent loads, not by bytes (a partial row is
+// 256-512 B): one thread per d walking the pieces four at a time took 24
+// round trips for the 94 pieces of one long sequence; eight waves of eight
+// loads take 64 pieces per round trip.  Up to 8 pieces are one round trip
+// of D threads, with no LDS and no barrier: a batch of mixed lengths has
+// about a thousand such rows, and eight waves for each cost 1.5 us more.
+constexpr int kMergeClasses = 8;
+constexpr int kMergeBatch = 8;
+
+template <bool BF16>
+__device__ __forceinline__ void merge_write(float M, float num, float den, int dd, uint16_t* orow,
+                                            float* lse) {
+  orow[dd] = f2h<BF16>(M != -INFINITY ? num / den : 0.f);
+  if (lse && dd == 0)
+    *lse = M != -INFINITY ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
+}
+
+template <bool BF16, int D, typename SlotOf>
 __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float* __restrict__ pl,
-                                             const float* __restrict__ po, int d, int dd,
-                                             float* M_out, float* num_out, float* den_out) {
-  constexpr int kBatch = 4;
-  float M = -INFINITY, num = 0.f, den = 0.f;
-  for (int s0 = 0; s0 < n; s0 += kBatch) {
-    float lv[kBatch], ov[kBatch];
+                                             const float* __restrict__ po, uint16_t* orow,
+                                             float* lse) {
+  constexpr int V = D / kWave;  // d per lane
+  const int dd = threadIdx.x;
+  if (n <= kMergeClasses) {
+    if (dd >= D) return;
+    float lv[kMergeClasses], ov[kMergeClasses];
+    float M = -INFINITY, den = 0.f, num = 0.f;
 #pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      lv[k] = -INFINITY;
-      ov[k] = 0.f;
-      if (s0 + k < n) {
-        const int64_t sh = slot_of(s0 + k);
-        lv[k] = pl[sh];
-        if (dd < d) ov[k] = po[sh * d + dd];
+    for (int s = 0; s < kMergeClasses; ++s) {
+      lv[s] = -INFINITY;
+      ov[s] = 0.f;
+      if (s < n) {
+        const int64_t sh = slot_of(s);
+        lv[s] = pl[sh];
+        ov[s] = po[sh * D + dd];
+      }
+      M = fmaxf(M, lv[s]);
+    }
+    if (M != -INFINITY) {
+#pragma unroll
+      for (int s = 0; s < kMergeClasses; ++s) {
+        const float wt = lv[s] == -INFINITY ? 0.f : exp2f(lv[s] - M);
+        den += wt;
+        num = fmaf(wt, ov[s], num);
       }
     }
-    float Mb = M;
-#pragma unroll
-    for (int k = 0; k < kBatch; ++k) Mb = fmaxf(Mb, lv[k]);
-    if (Mb == -INFINITY) continue;
-    const float r = M == -INFINITY ? 0.f : exp2f(M - Mb);
-    num *= r;
-    den *= r;
-#pragma unroll
-    for (int k = 0; k < kBatch; ++k) {
-      const float wt = lv[k] == -INFINITY ? 0.f : exp2f(lv[k] - Mb);
-      den += wt;
-      num += wt * ov[k];
-    }
-    M = Mb;
+    merge_write<BF16>(M, num, den, dd, orow, lse);
+    return;
   }
-  *M_out = M;
-  *num_out = num;
-  *den_out = den;
+  __shared__ float s_m[kMergeClasses], s_den[kMergeClasses], s_num[kMergeClasses][D];
+  const int wave = uniform(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  for (int cls = wave; cls < kMergeClasses; cls += blockDim.x >> 6) {
+    float M = -INFINITY, den = 0.f, num[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) num[e] = 0.f;
+    for (int s0 = cls; s0 < n; s0 += kMergeClasses * kMergeBatch) {
+      float lv[kMergeBatch], ov[kMergeBatch][V];
+#pragma unroll
+      for (int k = 0; k < kMergeBatch; ++k) {
+        const int s = s0 + kMergeClasses * k;
+        lv[k] = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < V; ++e) ov[k][e] = 0.f;
+        if (s < n) {
+          const int64_t sh = slot_of(s);
+          lv[k] = pl[sh];
+#pragma unroll
+          for (int e = 0; e < V; ++e) ov[k][e] = po[sh * D + V * lane + e];
+        }
+      }
+      float Mb = M;
+#pragma unroll
+      for (int k = 0; k < kMergeBatch; ++k) Mb = fmaxf(Mb, lv[k]);
+      if (Mb == -INFINITY) continue;
+      const float r = M == -INFINITY ? 0.f : exp2f(M - Mb);
+      den *= r;
+#pragma unroll
+      for (int e = 0; e < V; ++e) num[e] *= r;
+#pragma unroll
+      for (int k = 0; k < kMergeBatch; ++k) {
+        const float wt = lv[k] == -INFINITY ? 0.f : exp2f(lv[k] - Mb);
+        den += wt;
+#pragma unroll
+        for (int e = 0; e < V; ++e) num[e] = fmaf(wt, ov[k][e], num[e]);
+      }
+      M = Mb;
+    }
+    if (lane == 0) {
+      s_m[cls] = M;
+      s_den[cls] = den;
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) s_num[cls][V * lane + e] = num[e];
+  }
+  __syncthreads();
+  if (dd >= D) return;
+  float M = -INFINITY, den = 0.f, num = 0.f;
+#pragma unroll
+  for (int w = 0; w < kMergeClasses; ++w) M = fmaxf(M, s_m[w]);
+  if (M != -INFINITY) {
+#pragma unroll
+    for (int w = 0; w < kMergeClasses; ++w) {
+      const float wt = s_m[w] == -INFINITY ? 0.f : exp2f(s_m[w] - M);
+      den = fmaf(wt, s_den[w], den);
+      num = fmaf(wt, s_num[w][dd], num);
+    }
+  }
+  merge_write<BF16>(M, num, den, dd, orow, lse);
 }
 
 // Split-KV merge, one workgroup per (split group, query head):
@@ -1348,29 +1424,23 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
 // lse = M + log2(sum_c 2^(lse_c - M)) (base-2 partials, natural-log output).
 // A separate launch: the kernel boundary orders the partial writes before
 // these reads across the XCDs' L2 caches without per-item cache flushes.
-template <bool BF16>
-__global__ void __launch_bounds__(128)
+template <bool BF16, int D>
+__global__ void __launch_bounds__(kWave * kMergeClasses)
     decode_merge_kernel(const MergeItem* __restrict__ merges,
                         const float* __restrict__ po,
                         const float* __restrict__ pl, uint16_t* __restrict__ out,
-                        float* __restrict__ lse, int hq, int g, int d) {
+                        float* __restrict__ lse, int hq, int g) {
   const MergeItem mi = merges[blockIdx.x];
   const int hn = blockIdx.y;  // query head within the group
-  const int head = mi.h * g + hn;
-  const int dd = threadIdx.x;
-  float M, num, den;
-  merge_pieces(mi.nslots, [&](int s) { return (int64_t)(mi.slot0 + s * mi.stride) * g + hn; },
-               pl, po, d, dd, &M, &num, &den);
-  if (dd < d)
-    out[((int64_t)mi.b * hq + head) * d + dd] =
-        f2h<BF16>(M != -INFINITY ? num / den : 0.f);
-  if (lse && dd == 0)
-    lse[(int64_t)mi.b * hq + head] =
-        M != -INFINITY ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
+  const int64_t row = (int64_t)mi.b * hq + mi.h * g + hn;
+  merge_pieces<BF16, D>(
+      mi.nslots, [&](int s) { return (int64_t)(mi.slot0 + s * mi.stride) * g + hn; }, pl, po,
+      out + row * D, lse ? lse + row : nullptr);
 }
 
 // Split-KV merge of a device-side partition, one workgroup per (sequence,
-// KV head, query head of its group), one thread per d: the pieces of a cut (sequence, head group) segment sit in shares
+// KV head, query head of its group): the pieces of a cut (sequence, head
+// group) segment sit in shares
 // first..last; the piece in share w wrote slot (2 w + j) * hg + wi with j = 1
 // only for the first share when the segment starts inside it.  Empty
 // sequences get zero output and lse = -inf here (the attention launch has no
@@ -1381,11 +1451,12 @@ struct MergeImplicitArgs {
   const float* pl;
   uint16_t* out;
   float* lse;
-  int32_t batch, hq, hkv, g, d, hg_shift, n_groups, item_cost;
+  int32_t batch, hq, hkv, g, hg_shift, n_groups, item_cost;
 };
 
-template <bool BF16>
-__global__ void __launch_bounds__(128) decode_merge_implicit_kernel(MergeImplicitArgs a) {
+template <bool BF16, int D>
+__global__ void __launch_bounds__(kWave * kMergeClasses)
+    decode_merge_implicit_kernel(MergeImplicitArgs a) {
   const int b = blockIdx.x / a.hkv;
   const int h = blockIdx.x % a.hkv;
   const int hn = blockIdx.y;  // query head within the group
@@ -1395,9 +1466,9 @@ __global__ void __launch_bounds__(128) decode_merge_implicit_kernel(MergeImplici
   const ImplicitSplit sp = implicit_split(a.kv_indptr, a.batch, ngrp, a.n_groups, a.item_cost);
   const int ind_lo = load_invariant(a.kv_indptr + b);
   const int np = load_invariant(a.kv_indptr + b + 1) - ind_lo;
-  uint16_t* orow = a.out + ((int64_t)b * a.hq + head) * a.d;
+  uint16_t* orow = a.out + ((int64_t)b * a.hq + head) * D;
   if (np <= 0) {
-    if (dd < a.d) orow[dd] = f2h<BF16>(0.f);
+    if (dd < D) orow[dd] = f2h<BF16>(0.f);
     if (a.lse && dd == 0) a.lse[(int64_t)b * a.hq + head] = -INFINITY;
     return;
   }
@@ -1412,13 +1483,9 @@ __global__ void __launch_bounds__(128) decode_merge_implicit_kernel(MergeImplici
     const int j = (w == first && p0 != w * sp.share) ? 1 : 0;
     return ((2 * w + j) << a.hg_shift) + wi;
   };
-  float M, num, den;
-  merge_pieces((int)(last - first + 1), [&](int s) { return slot_of(first + s) * a.g + hn; },
-               a.pl, a.po, a.d, dd, &M, &num, &den);
-  if (dd < a.d) orow[dd] = f2h<BF16>(M != -INFINITY ? num / den : 0.f);
-  if (a.lse && dd == 0)
-    a.lse[(int64_t)b * a.hq + head] =
-        M != -INFINITY ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
+  merge_pieces<BF16, D>(
+      (int)(last - first + 1), [&](int s) { return slot_of(first + s) * a.g + hn; }, a.pl, a.po,
+      orow, a.lse ? a.lse + (int64_t)b * a.hq + head : nullptr);
 }
 
 // ----------------------------------------------------------------------------
@@ -1595,26 +1662,28 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
   if (rc) return rc;
   if (plan->implicit) {
     MergeImplicitArgs m{kv_indptr, plan->partial_o, plan->partial_lse, p.out, lse,
-                        plan->batch_size, plan->hq, plan->hkv, p.g, plan->d,
+                        plan->batch_size, plan->hq, plan->hkv, p.g,
                         plan->hg_shift, plan->n_items, plan->item_cost};
     const dim3 grid((unsigned)((int64_t)plan->batch_size * plan->hkv), p.g);
-    if (bf16)
-      hipLaunchKernelGGL(decode_merge_implicit_kernel<true>, grid, dim3(plan->d), 0, s, m);
-    else
-      hipLaunchKernelGGL(decode_merge_implicit_kernel<false>, grid, dim3(plan->d), 0, s, m);
+    auto* mfn = plan->d == 64 ? (bf16 ? decode_merge_implicit_kernel<true, 64>
+                                      : decode_merge_implicit_kernel<false, 64>)
+                              : (bf16 ? decode_merge_implicit_kernel<true, 128>
+                                      : decode_merge_implicit_kernel<false, 128>);
+    // piece counts are only known on the device: eight waves a row while the
+    // rows are too few to fill the GPU by themselves
+    const int64_t rows = (int64_t)plan->batch_size * plan->hq;
+    hipLaunchKernelGGL(mfn, grid, dim3(rows <= 1024 ? kWave * kMergeClasses : plan->d), 0, s, m);
     return check_launch("decode_run(merge)");
   }
   if (plan->n_merge == 0) return rc;
   const dim3 grid(plan->n_merge, p.g);
-  const MergeItem* merges = static_cast<const MergeItem*>(plan->merge_dev);
-  if (bf16)
-    hipLaunchKernelGGL(decode_merge_kernel<true>, grid, dim3(plan->d), 0, s, merges,
-                       plan->partial_o, plan->partial_lse, p.out, lse, plan->hq, p.g,
-                       plan->d);
-  else
-    hipLaunchKernelGGL(decode_merge_kernel<false>, grid, dim3(plan->d), 0, s, merges,
-                       plan->partial_o, plan->partial_lse, p.out, lse, plan->hq, p.g,
-                       plan->d);
+  auto* mfn = plan->d == 64
+                  ? (bf16 ? decode_merge_kernel<true, 64> : decode_merge_kernel<false, 64>)
+                  : (bf16 ? decode_merge_kernel<true, 128> : decode_merge_kernel<false, 128>);
+  hipLaunchKernelGGL(mfn, grid,
+                     dim3(plan->max_pieces > kMergeClasses ? kWave * kMergeClasses : plan->d), 0, s,
+                     static_cast<const MergeItem*>(plan->merge_dev), plan->partial_o,
+                     plan->partial_lse, p.out, lse, plan->hq, p.g);
   return check_launch("decode_run(merge)");
 }
 

@@ -57,9 +57,16 @@ static int decode_head_group(int hkv) {
 // PAGEDATTN_DECODE_SHARED_SLACK_KB KiB (default 96: what one CU streams in
 // the 4-5 us that the split's merge launch costs) plus
 // PAGEDATTN_DECODE_SHARED_SLACK_PCT percent of the mean (default 4: the
-// split's partials and per-item restarts) more K/V than the mean.  Measured
-// on the 70B-shaped e4m3 batch (D = 128, busiest CU 3.1 % over the mean):
-// 214 us shared against 225 us split.
+// split's partials and per-item restarts) more K/V than the mean over all
+// CUs.  Measured on the 70B-shaped e4m3 batch (D = 128, busiest CU 3.1 % over
+// the mean): 214 us shared against 225 us split.  Batches of fewer items than
+// CUs leave CUs idle, and the busy ones then stream faster (38 against 26
+// KiB/us each), so their default slack is 120 KiB: equal-length sequences of
+// 128 KiB an item run 8.7-8.9 us either way on 8-64 items (the split's second
+// launch on top where the host launches each step), and 256 KiB an item 10.8
+// us shared against 9.4 us split on 8 items, 14.0 against 12.5 us on 128.
+// One sequence of 9001 tokens over 8 KV heads of D = 128 (4.4 MiB an item on
+// 8 of 256 CUs): 93 us shared, 14 us split.
 static int decode_shared_mode() {
   if (const char* env = std::getenv("PAGEDATTN_DECODE_SHARED")) {
     const int v = std::atoi(env);
@@ -86,12 +93,12 @@ static bool shared_xcd_affine() {
   return !(env && std::atoi(env) == 0);
 }
 
-static int64_t decode_shared_slack_bytes() {
+static int64_t decode_shared_slack_bytes(bool idle_cus) {
   if (const char* env = std::getenv("PAGEDATTN_DECODE_SHARED_SLACK_KB")) {
     const int v = std::atoi(env);
     if (v >= 0) return (int64_t)v << 10;
   }
-  return (int64_t)96 << 10;
+  return (int64_t)(idle_cus ? 120 : 96) << 10;
 }
 static int decode_shared_slack_pct() {
   if (const char* env = std::getenv("PAGEDATTN_DECODE_SHARED_SLACK_PCT")) {
@@ -110,15 +117,19 @@ static int decode_shared_slack_pct() {
 // and one chunk over a multiple of four costs a whole round.  (On the
 // 70B-shaped e4m3 batch the busiest of 256 workgroups goes from 606 to about
 // 590 chunks, 213 -> 210 us.)
-// Returns false (and leaves the outputs unspecified) when some workgroup
+// Returns kSharedNo (and leaves the outputs unspecified) when some workgroup
 // would hold more than kSharedMaxItems items or, unless forced, when the
-// busiest workgroup exceeds the mean by more than the slack.
-static bool plan_shared(const std::vector<int32_t>& npages, const int32_t* kv_indptr_host,
+// busiest workgroup exceeds the mean by more than the slack; kSharedFallback
+// when only the CUs left idle make it exceed the mean: the split partition
+// is then faster, and this one stands in where the workspace cannot hold the
+// split's partials.
+enum SharedFit { kSharedNo, kSharedFallback, kSharedYes };
+static SharedFit plan_shared(const std::vector<int32_t>& npages, const int32_t* kv_indptr_host,
                         const int32_t* kv_last_page_len_host, int hkv, int d, int cus,
                         bool forced, std::vector<SharedItem>* items, int* n_wg_out) {
   const int batch = (int)npages.size();
   const int64_t n_all = (int64_t)batch * hkv;
-  if (n_all == 0) return false;
+  if (n_all == 0) return kSharedNo;
   const int chunk_pages = 2 * kSharedStagePairs;
   auto chunks_of = [&](int32_t id) {
     const int32_t np = npages[id / hkv];
@@ -306,17 +317,22 @@ static bool plan_shared(const std::vector<int32_t>& npages, const int32_t* kv_in
   }
   int64_t sum = 0, mx = 0;
   for (int w = 0; w < n_wg; ++w) {
-    if ((int)per[w].size() > kSharedMaxItems) return false;
+    if ((int)per[w].size() > kSharedMaxItems) return kSharedNo;
     sum += load[w];
     mx = std::max(mx, load[w]);
   }
   // K and V of one page of one KV head, counted at 16 bits per element
   const int64_t page_bytes = (int64_t)kPage * d * 2 * 2;
-  // busiest - mean > slack + pct% of the mean, scaled by n_wg
-  if (!forced && (mx * n_wg - sum) * page_bytes * 100 >
-                     decode_shared_slack_bytes() * n_wg * 100 +
-                         sum * page_bytes * decode_shared_slack_pct())
-    return false;
+  // busiest - mean > slack + pct% of the mean, scaled by the workgroups or
+  // CUs the mean is over
+  auto over = [&](int64_t n, int64_t slack) {
+    return (mx * n - sum) * page_bytes * 100 >
+           slack * n * 100 + sum * page_bytes * decode_shared_slack_pct();
+  };
+  const int64_t n_cus = std::max(cus, 1);
+  const bool idle_cus = n_wg < n_cus;
+  if (!forced && over(n_wg, decode_shared_slack_bytes(false))) return kSharedNo;
+  const bool fallback = !forced && idle_cus && over(n_cus, decode_shared_slack_bytes(true));
   // fixed stride: workgroup w's items at [w kSharedMaxItems, ...), padded
   items->assign((size_t)n_wg * kSharedMaxItems, SharedItem{-1, 0, 0, 0, -1, 0, kPage, 0});
   for (int w = 0; w < n_wg; ++w) {
@@ -335,7 +351,7 @@ static bool plan_shared(const std::vector<int32_t>& npages, const int32_t* kv_in
     }
   }
   *n_wg_out = n_wg;
-  return true;
+  return fallback ? kSharedFallback : kSharedYes;
 }
 
 // The device-side partition of a decode plan (pagedattn_decode_plan_device
@@ -427,46 +443,48 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
   plan->shared = false;
   plan->dev_table = false;
 
-  if (split_pages == 0 && decode_shared_mode() != 0) {
-    std::vector<SharedItem> sitems;
-    int n_wg = 0;
-    if (plan_shared(npages, kv_indptr_host, kv_last_page_len_host, hkv, head_dim, cus,
-                    decode_shared_mode() == 1, &sitems, &n_wg)) {
-      const size_t off_items = kWsHeader;
-      const size_t end = ws_align(off_items + sizeof(SharedItem) * sitems.size());
-      const size_t host_bytes = end - kWsHeader;
-      plan->host.assign(host_bytes / sizeof(int32_t), 0);
-      char* hb = reinterpret_cast<char*>(plan->host.data());
-      std::memcpy(hb, sitems.data(), sizeof(SharedItem) * sitems.size());
-      plan->workspace = workspace;
-      plan->workspace_bytes = workspace_bytes;
-      rc = upload_plan(plan, who, host_bytes, end, stream);
-      if (rc) return rc;
-      char* ws = static_cast<char*>(workspace);
-      plan->implicit = false;
-      plan->shared = true;
-      plan->deterministic = decode_deterministic();
-      plan->batch_size = batch_size;
-      plan->hq = num_qo_heads;
-      plan->hkv = num_kv_heads;
-      plan->d = head_dim;
-      plan->page_size = page_size;
-      plan->n_items = n_wg;
-      plan->hg_shift = 0;
-      plan->n_merge = 0;
-      plan->n_slots = 0;
-      plan->split_pages = split_pages;
-      plan->items_dev = ws + off_items;
-      plan->wave_ptr_dev = nullptr;
-      plan->merge_dev = nullptr;
-      plan->partial_o = nullptr;
-      plan->partial_lse = nullptr;
-      plan->total_pages = total;
-      plan->max_pages = maxp;
-      plan->mode = kPlanDecode;
-      return PAGEDATTN_OK;
-    }
-  }
+  std::vector<SharedItem> sitems;
+  int n_wg = 0;
+  SharedFit fit = kSharedNo;
+  if (split_pages == 0 && decode_shared_mode() != 0)
+    fit = plan_shared(npages, kv_indptr_host, kv_last_page_len_host, hkv, head_dim, cus,
+                      decode_shared_mode() == 1, &sitems, &n_wg);
+  auto use_shared = [&]() -> int {
+    const size_t off_items = kWsHeader;
+    const size_t end = ws_align(off_items + sizeof(SharedItem) * sitems.size());
+    const size_t host_bytes = end - kWsHeader;
+    plan->host.assign(host_bytes / sizeof(int32_t), 0);
+    char* hb = reinterpret_cast<char*>(plan->host.data());
+    std::memcpy(hb, sitems.data(), sizeof(SharedItem) * sitems.size());
+    plan->workspace = workspace;
+    plan->workspace_bytes = workspace_bytes;
+    const int rc = upload_plan(plan, who, host_bytes, end, stream);
+    if (rc) return rc;
+    char* ws = static_cast<char*>(workspace);
+    plan->implicit = false;
+    plan->shared = true;
+    plan->deterministic = decode_deterministic();
+    plan->batch_size = batch_size;
+    plan->hq = num_qo_heads;
+    plan->hkv = num_kv_heads;
+    plan->d = head_dim;
+    plan->page_size = page_size;
+    plan->n_items = n_wg;
+    plan->hg_shift = 0;
+    plan->n_merge = 0;
+    plan->n_slots = 0;
+    plan->split_pages = split_pages;
+    plan->items_dev = ws + off_items;
+    plan->wave_ptr_dev = nullptr;
+    plan->merge_dev = nullptr;
+    plan->partial_o = nullptr;
+    plan->partial_lse = nullptr;
+    plan->total_pages = total;
+    plan->max_pages = maxp;
+    plan->mode = kPlanDecode;
+    return PAGEDATTN_OK;
+  };
+  if (fit == kSharedYes) return use_shared();
 
   // work is planned per head group: hg KV heads walked together by hg waves
   const int hg = decode_head_group(hkv);
@@ -618,6 +636,8 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
       ws_align(off_po + sizeof(float) * (size_t)n_slots * g * head_dim);
   const size_t end = ws_align(off_pl + sizeof(float) * (size_t)n_slots * g);
   const size_t host_bytes = off_po - kWsHeader;
+  // a small batch whose partials do not fit stays whole
+  if (fit == kSharedFallback && end > workspace_bytes) return use_shared();
 
   plan->host.assign(host_bytes / sizeof(int32_t), 0);
   char* hb = reinterpret_cast<char*>(plan->host.data());
@@ -642,6 +662,7 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
   plan->n_items = n_waves;
   plan->hg_shift = hg_shift;
   plan->n_merge = (int)n_merge;
+  plan->max_pieces = pieces.empty() ? 0 : *std::max_element(pieces.begin(), pieces.end());
   plan->n_slots = n_slots;
   plan->split_pages = split_pages;
   plan->items_dev = ws + off_items;

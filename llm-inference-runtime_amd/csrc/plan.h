@@ -89,6 +89,8 @@ struct pagedattn_plan {
   int batch_size = 0, hq = 0, hkv = 0, d = 0, page_size = 0;
   // n_items = head groups (decode) or work items (prefill)
   int n_items = 0, n_merge = 0, n_slots = 0, split_pages = 0;
+  // decode, split: most pieces any (sequence, head group) was cut in
+  int max_pieces = 0;
   // decode: log2 of the waves (KV heads) per head group
   int hg_shift = 0;
   // decode: the partition is made on the device at run time from kv_indptr

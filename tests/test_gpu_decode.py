@@ -68,6 +68,52 @@ def test_decode_balanced_item_cost(gpu, monkeypatch, cost):
     assert lse_err(lse, ref_l) <= TOL_LSE
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("pieces", [[8, 3, 1], [9, 8, 2], [16, 17], [63, 65, 1]])
+def test_decode_merge_piece_counts(gpu, d, pieces):
+    # fixed chunks of 128 tokens: up to 8 pieces a row (one round trip of the
+    # merge), one past it, and around its 64 pieces per round trip
+    lens = [128 * n - (5 if n > 1 else 100) for n in pieces]
+    meta, pool, q = decode_case(gpu, lens, 16, 2, d, seed=sum(pieces))
+    ref_o, ref_l = oracle_decode(meta, pool, q)
+    out, lse = run_decode(gpu, meta, pool, q, 16, 2, d, split_pages=8)
+    assert max_err(out, ref_o) <= TOL_BF16
+    assert lse_err(lse, ref_l) <= TOL_LSE
+
+
+@pytest.mark.parametrize("lens,hq", [([9001], 16), ([9001] + [20] * 69, 16)])
+def test_decode_device_plan_one_long_sequence(gpu, lens, hq):
+    # the device partition's merge over many pieces, with eight waves a row
+    # (few rows) and with D threads a row (more than 1024 rows)
+    meta, pool, q = decode_case(gpu, lens, hq, 2, 128, seed=len(lens))
+    ref_o, ref_l = oracle_decode(meta, pool, q)
+    w = pagedattn.BatchDecodeWithPagedKVCacheWrapper(workspace(gpu), "HND")
+    w.plan(i32(meta.kv_indptr, gpu), i32(meta.kv_indices, gpu),
+           i32(meta.kv_last_page_len, gpu), hq, 2, 128, 16, q_data_type=q.dtype,
+           device_plan=True)
+    out, lse = w.run(q, pool, return_lse=True)
+    assert max_err(out, ref_o) <= TOL_BF16
+    assert lse_err(lse, ref_l) <= TOL_LSE
+
+
+def test_decode_few_items_split_where_the_workspace_allows(gpu, monkeypatch):
+    # two long items on an idle GPU are cut; with a workspace that cannot hold
+    # the partials they run whole, as they always did
+    for var in ("PAGEDATTN_DECODE_SHARED", "PAGEDATTN_DECODE_SHARED_SLACK_KB"):
+        monkeypatch.delenv(var, raising=False)
+    meta, pool, q = decode_case(gpu, [3000], 16, 2, 128, seed=1)
+    ref_o, ref_l = oracle_decode(meta, pool, q)
+    for size, kind in ((1 << 22, "split"), (1 << 13, "shared")):
+        w = pagedattn.BatchDecodeWithPagedKVCacheWrapper(
+            torch.zeros(size, dtype=torch.uint8, device=gpu), "HND")
+        w.plan(i32(meta.kv_indptr, gpu), i32(meta.kv_indices, gpu),
+               i32(meta.kv_last_page_len, gpu), 16, 2, 128, 16, q_data_type=q.dtype)
+        assert w.plan_kind == kind
+        out, lse = w.run(q, pool, return_lse=True)
+        assert max_err(out, ref_o) <= TOL_BF16
+        assert lse_err(lse, ref_l) <= TOL_LSE
+
+
 def test_decode_fp16(gpu):
     meta, pool, q = decode_case(gpu, EDGE_LENS, 32, 4, 64, dtype=torch.float16, seed=11)
     ref_o, ref_l = oracle_decode(meta, pool, q)
