@@ -246,7 +246,11 @@ int pagedattn_build_paged_metadata(const int32_t* block_tables, int64_t table_st
  * gave up (never in a consistent run: the item's output is then left
  * unwritten rather than merged wrongly); byte 12, q-tiles that device-planned
  * prefill runs dropped because they exceeded the plan's capacity (their
- * output rows are left unwritten). */
+ * output rows are left unwritten).
+ *
+ * Runs whose plan cuts KV ranges write their split partials into the
+ * workspace, so two runs of one plan must not overlap on the GPU (runs of
+ * one stream never do); give concurrent streams a plan and a workspace each. */
 pagedattn_plan* pagedattn_plan_create(void);
 void pagedattn_plan_destroy(pagedattn_plan* plan);
 
@@ -311,9 +315,11 @@ int pagedattn_decode_plan_device_update(pagedattn_plan* plan, const int32_t* kv_
  * at run time, see pagedattn_decode_plan_device), or 0
  * for a plan that is not a decode plan.  pagedattn_decode_plan with
  * split_pages = 0 takes a shared plan when its busiest CU carries at most
- * PAGEDATTN_DECODE_SHARED_SLACK_KB (environment, default 96) KiB plus
- * PAGEDATTN_DECODE_SHARED_SLACK_PCT (default 4) percent of the mean more K/V
- * than the mean; PAGEDATTN_DECODE_SHARED=0 / =1 turns that off / takes one
+ * PAGEDATTN_DECODE_SHARED_SLACK_KB (environment, default 96, or 120 for fewer
+ * items than CUs) KiB plus PAGEDATTN_DECODE_SHARED_SLACK_PCT (default 4)
+ * percent of the mean more K/V than the mean over all CUs (a workspace too
+ * small for the split's partials keeps a plan that is balanced over the CUs
+ * it uses); PAGEDATTN_DECODE_SHARED=0 / =1 turns that off / takes one
  * whenever it fits.  A shared plan's waves take fixed page pairs, so repeated
  * runs give identical bits; PAGEDATTN_DECODE_DETERMINISTIC=0 (read at plan
  * time) lets them claim pairs in arrival order instead, which balances the
@@ -392,7 +398,11 @@ int pagedattn_decode_run_rope_append(
  *     (src/models/llama.py:86-116).  Host copies of the indptr arrays.
  * q-tiles of at most half a workgroup's rows are planned as pairs of KV
  * heads sharing one workgroup when num_kv_heads is even (same output bits);
- * PAGEDATTN_PREFILL_PAIR=0, read at plan time, plans every tile alone. */
+ * PAGEDATTN_PREFILL_PAIR=0, read at plan time, plans every tile alone.
+ * Steps with fewer q-tiles x KV heads than CUs cut the KV range of their long
+ * tiles into pieces merged by a second launch, where the workspace holds the
+ * partials (about 34 MiB at 256 CUs and D = 128, half at D = 64);
+ * PAGEDATTN_PREFILL_SPLIT=0, read at plan time, keeps every tile whole. */
 int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
                            const int32_t* kv_indptr_host,
                            const int32_t* kv_last_page_len_host,
@@ -408,11 +418,13 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
  * (max_qo_tokens, the sum of the qo lengths) are fixed here.  Every
  * pagedattn_prefill_run with this plan first launches one workgroup that
  * cuts the q-tiles of the run's qo_indptr / kv_indptr / kv_last_page_len
- * exactly as pagedattn_prefill_plan does (same pairing, up to 1024 tiles
- * ordered longest first), into the workspace, then the attention over the
- * plan's fixed capacity of ceil(max_qo_tokens / q_tile) + batch_size tiles;
- * entries past the run's tiles return at once.  The outputs equal those of
- * a host plan bit for bit.  Tiles beyond the capacity (a run with more than
+ * exactly as pagedattn_prefill_plan does (same pairing and pieces, up to 1024
+ * tiles ordered longest first), into the workspace, then the attention over
+ * the plan's fixed capacity of ceil(max_qo_tokens / q_tile) + batch_size tiles
+ * (at least one workgroup per CU where pieces may be cut, and then the merge
+ * launch); entries past the run's tiles return at once.  The outputs equal
+ * those of a host plan bit for bit (whose workspace, like this one, holds the
+ * partials, or does not).  Tiles beyond the capacity (a run with more than
  * max_qo_tokens query tokens) are skipped and counted at byte 12 of the
  * workspace.  batch_size <= 4096. */
 int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,

@@ -40,6 +40,19 @@ struct PrefillItem {
   int32_t b, q_lo, q_hi, slot;
 };
 
+// One entry of a split prefill work list: piece k of the n that the KV tiles
+// of query tokens [q_lo, q_hi) of sequence b are cut into (prefill_pieces).
+// n = 1: the whole tile, written to the output (`flag` as PrefillItem::slot);
+// n > 1: split partials to slot `slot` of every KV head.
+struct PrefillPiece {
+  int32_t b, q_lo, q_hi, flag, k, n, slot, pad;
+};
+
+// A cut q-tile: its pieces hold slots [slot0, slot0 + n).
+struct PrefillMerge {
+  int32_t b, q_lo, q_hi, slot0, n, pad0, pad1, pad2;
+};
+
 // One item of a shared-item decode plan (decode_shared_kernel): sequence b,
 // KV head h, its page pairs being chunks [chunk_lo, chunk_lo + n_chunks) of
 // the workgroup's chunk sequence; the sequence's pages are kv_indices
@@ -74,6 +87,35 @@ constexpr int kPrefillRows = kPrefillWaves * 32 * kPrefillRB;
 // (one rank each per thread; beyond this the tiles keep sequence order).
 constexpr int kPrefillDevMaxBatch = 4096;
 constexpr int kPrefillDevSortMax = 1024;
+// Split-KV prefill: a step whose q-tiles x KV heads are fewer than the CUs
+// cuts the KV tiles of its long q-tiles into pieces, one workgroup each, merged
+// by a second launch.  The longest tile of t_max KV tiles gets P pieces of
+// ceil(t_max / P), every other tile pieces of at most that many: P is the
+// largest (up to kPrefillSplitMaxPieces) whose pieces all run at once, with
+// at least kPrefillSplitMinTiles KV tiles a piece.
+constexpr int kPrefillSplitMaxPieces = 128;
+constexpr int kPrefillSplitMinTiles = 4;
+constexpr int kPrefillKvTile = 64;
+// Whether pieces of at most `len` KV tiles, `pieces` of them on `slots` places
+// per KV head, beat the longest workgroup's t_max: a KV tile takes 1.5 us on a
+// mostly idle GPU and 2 us on a full one, and the partials and the merge
+// launch 5 us plus 6 us on a full GPU (D = 128; at D = 64 all of it is about
+// a third less).  Measured on steps of 32/8 heads, D = 128, one tile per
+// sequence unless stated: 1 x 8 workgroups of 16 KV tiles 30.7 us whole, 12.5
+// us cut; 8 x 8 of 13 28.7 and 24.8 us, of 133 200 and 85 us; 16 x 8 of 17
+// 38.5 and 41.7 us (kept whole), of 24 45.7 and 44.7 us, of 141 212 and 157 us.
+inline __host__ __device__ bool prefill_split_pays(int t_max, int len, int64_t pieces,
+                                                   int64_t slots) {
+  return t_max - len >= 6 &&
+         3 * slots * t_max > (3 * slots + pieces) * len + 10 * slots + 12 * pieces;
+}
+
+// Workspace of a split prefill plan, from the workspace start: the cut tiles'
+// count, `entries` work-list entries, the merge list and the partials of
+// `slots` slots of every KV head.
+struct PrefillSplitLayout {
+  size_t off_count, off_pieces, off_merges, off_po, off_pl, end;
+};
 
 // Workspace layout: [0, kWsHeader) is reserved for the caller's device flags
 // (the Python shim keeps the append error counter at offset 0).
@@ -81,6 +123,18 @@ constexpr size_t kWsHeader = 256;
 constexpr size_t kWsAlign = 256;
 
 inline size_t ws_align(size_t x) { return (x + kWsAlign - 1) & ~(kWsAlign - 1); }
+
+inline PrefillSplitLayout prefill_split_layout(int64_t entries, int64_t slots, int hkv, int d) {
+  PrefillSplitLayout l;
+  l.off_count = kWsHeader;
+  l.off_pieces = l.off_count + kWsAlign;
+  l.off_merges = ws_align(l.off_pieces + sizeof(PrefillPiece) * (size_t)entries);
+  l.off_po = ws_align(l.off_merges + sizeof(PrefillMerge) * (size_t)(slots / 2 + 1));
+  const size_t rows = (size_t)slots * hkv * kPrefillRows;
+  l.off_pl = ws_align(l.off_po + sizeof(float) * rows * d);
+  l.end = ws_align(l.off_pl + sizeof(float) * rows);
+  return l;
+}
 
 }  // namespace pa
 
@@ -117,6 +171,11 @@ struct pagedattn_plan {
   // prefill: tiles of at most half a workgroup's rows run as KV-head pairs
   // (device plans apply it at run time; host plans flag their items)
   bool prefill_pair = false;
+  // prefill: the work list is one of PrefillPiece entries with a merge list
+  // and n_slots partial slots per KV head (host plans: some tile is cut;
+  // device plans: the plan kernel may cut tiles)
+  bool prefill_split = false;
+  int q_cap = 0;  // device plans that may cut tiles: q-tiles the plan holds
   int64_t total_qo = 0;
   // device pointers into the workspace
   void* items_dev = nullptr;

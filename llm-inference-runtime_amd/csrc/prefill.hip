@@ -24,6 +24,10 @@
 // page's valid tokens: absent pages and slots past last_page_len read as
 // zero without touching memory.  Causal tiles entirely below the diagonal
 // skip masking; tiles above the last row's diagonal are never visited.
+//
+// Steps of few tiles (a 512-token chunk of a 32/8-head layer is 8 x 8
+// workgroups on 256 CUs) cut each tile's KV range into pieces, one workgroup
+// each (SPLIT), merged by a second launch (prefill_merge_kernel).
 #include <algorithm>
 #include <cfloat>
 #include <climits>
@@ -38,7 +42,7 @@
 namespace pa {
 
 struct PrefillParams {
-  const PrefillItem* items;
+  const void* items;  // PrefillItem, or PrefillPiece (SPLIT)
   int32_t n_items, batch_size;
   const uint16_t* q;
   int64_t q_sn, q_sh;
@@ -54,6 +58,13 @@ struct PrefillParams {
   float* lse;     // [nnz, hq] or null
   int32_t hq, hkv, g, causal;
   float scale_log2;
+  // SPLIT: partials of slot s, KV head h and 32-row block w, at block
+  // (s hkv + h) kPrefillRows / 32 + w: O / l in accumulator order
+  // [D / 32][4][64 lanes][4], so stores and loads are whole 1 KiB runs, and
+  // the rows' base-2 log-sum-exps [32]
+  float* partial_o;
+  float* partial_lse;
+  int32_t n_slots;
 };
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -270,7 +281,7 @@ __device__ __forceinline__ float lane_value(float v, int i) {
 // rescale of O and l runs on few tiles.
 constexpr float kRescaleSlack = 8.f;
 
-template <int D, bool BF16, bool FP8, int RB>
+template <int D, bool BF16, bool FP8, int RB, bool SPLIT>
 __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillParams p) {
   using C = PrefillCfg<D, BF16, FP8, RB>;
   constexpr int BN = C::BN;
@@ -302,7 +313,8 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
   // a work list that does not match this launch is skipped, never followed
   // (every condition is uniform over the workgroup)
   if (item >= p.n_items) return;
-  const int32_t* itp = reinterpret_cast<const int32_t*>(p.items + item);
+  constexpr int ITEM_INTS = (SPLIT ? sizeof(PrefillPiece) : sizeof(PrefillItem)) / 4;
+  const int32_t* itp = static_cast<const int32_t*>(p.items) + (int64_t)item * ITEM_INTS;
   const int b = uniform(load_invariant(itp + 0));
   if (b < 0 || b >= p.batch_size) return;
   const int qo_start = uniform(load_invariant(p.qo_indptr + b));
@@ -320,6 +332,17 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
   const int clean_end =
       p.causal ? min(kv_len, max(0, diag + q_lo + 1)) : kv_len;
   const int n_tiles = (kv_end + BN - 1) / BN;
+  // the KV tiles [t_lo, t_hi) of this workgroup: all of them, or piece k of n
+  int t_lo = 0, t_hi = n_tiles, slot = -1;
+  if constexpr (SPLIT) {
+    const int k = uniform(load_invariant(itp + 4));
+    const int n = uniform(load_invariant(itp + 5));
+    slot = uniform(load_invariant(itp + 6));
+    if (n < 1 || k < 0 || k >= n || slot >= p.n_slots || (n > 1) != (slot >= 0)) return;
+    const int each = n_tiles / n, rest = n_tiles % n;
+    t_lo = each * k + min(k, rest);
+    t_hi = t_lo + each + (k < rest ? 1 : 0);
+  }
   // A paired tile (flagged by the planner; at most half the workgroup's rows)
   // is run for KV heads h0 = h & ~1 and h0 + 1 by one workgroup of the pair,
   // the even head's (flag 1) or the odd head's (flag 2): waves
@@ -328,7 +351,7 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
   // every barrier.  The pair's other workgroup has nothing left to do.
   const int pflag = uniform(load_invariant(itp + 3));
   const bool paired = PAIRS && (p.hkv & 1) == 0 && (pflag == 1 || pflag == 2) &&
-                      (q_hi - q_lo) * g <= C::ROWS / 2;
+                      (q_hi - q_lo) * g <= C::ROWS / 2 && slot < 0;
   if (paired && (h & 1) != pflag - 1) return;
 
   // The tile loop of one head group: NW waves, wave index `wave` within the
@@ -392,18 +415,18 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
 
     HalfRegs<D, BF16, FP8, RB> kr, vr;  // e4m3 staging only
     float ksc_l = 0.f, vsc_l = 0.f;     // e4m3 scales of the computed tile
-    int pid = fetch_page_ids(p, ind_lo, npages, 0, lane);
-    if (n_tiles > 0) {
+    int pid = fetch_page_ids(p, ind_lo, npages, t_lo, lane);
+    if (t_lo < t_hi) {
       if constexpr (FP8) {
-        load_half<D, BF16, FP8, RB, false>(kr, p, h, pid, npages, last, 0, wave, lane);
-        load_half<D, BF16, FP8, RB, true>(vr, p, h, pid, npages, last, 0, wave, lane);
+        load_half<D, BF16, FP8, RB, false>(kr, p, h, pid, npages, last, t_lo, wave, lane);
+        load_half<D, BF16, FP8, RB, true>(vr, p, h, pid, npages, last, t_lo, wave, lane);
       } else {
-        dma_half<D, BF16, FP8, RB, false, NW>(p, h, pid, npages, last, 0, st0, wave, lane);
-        dma_half<D, BF16, FP8, RB, true, NW>(p, h, pid, npages, last, 0, st0 + C::TILEB,
+        dma_half<D, BF16, FP8, RB, false, NW>(p, h, pid, npages, last, t_lo, st0, wave, lane);
+        dma_half<D, BF16, FP8, RB, true, NW>(p, h, pid, npages, last, t_lo, st0 + C::TILEB,
                                              wave, lane);
       }
     }
-    int pid_next = fetch_page_ids(p, ind_lo, npages, 1, lane);
+    int pid_next = fetch_page_ids(p, ind_lo, npages, t_lo + 1, lane);
 
     // Tile t's QK, softmax and PV from stage `cur` (e4m3: with the register
     // loads of tile t + 1, pages pid_ld, issued between its phases).
@@ -547,7 +570,7 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
       __syncthreads();
       pid = pid_next;
       pid_next = fetch_page_ids(p, ind_lo, npages, t + 2, lane);
-      const int pid_ld = t + 1 < n_tiles ? pid : -1;  // past the last tile: no pages
+      const int pid_ld = t + 1 < t_hi ? pid : -1;  // past the last tile: no pages
       if constexpr (!FP8) {
         // tile t + 1 straight into the other stage, K and V, a whole tile
         // ahead of the barrier that waits for it
@@ -555,18 +578,19 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
         dma_half<D, BF16, FP8, RB, true, NW>(p, h, pid_ld, npages, last, t + 1, nxt + C::TILEB,
                                              wave, lane);
       }
-      // paired tiles: a wave with no row of the tile only loads
-      if (!decltype(pair_tag)::value || wave_rows) compute(mask_tag, t, cur, pid_ld);
+      // paired tiles and pieces: a wave with no row of the tile only loads
+      // (e4m3 pools: the loads are inside compute)
+      if (FP8 || (!decltype(pair_tag)::value && !SPLIT) || wave_rows) compute(mask_tag, t, cur, pid_ld);
     };
 
 
     // tiles [0, n_clean) lie wholly at or below the first row's diagonal
     // (and inside the sequence): no mask; the rest are masked.  Tile t uses
-    // stage t & 1 (the prologue loaded tile 0 into stage 0).
-    const int n_clean = min(n_tiles, clean_end / BN);
-    int t = 0;
+    // stage (t - t_lo) & 1 (the prologue loaded tile t_lo into stage 0).
+    const int n_clean = min(t_hi, SPLIT ? max(t_lo, clean_end / BN) : clean_end / BN);
+    int t = t_lo;
     auto run_tiles = [&](auto mask_tag, const int t_end) __attribute__((always_inline)) {
-      if (t < t_end && (t & 1)) {
+      if (t < t_end && ((t - t_lo) & 1)) {
         step(mask_tag, t, st1, st0);
         ++t;
       }
@@ -580,7 +604,7 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
       }
     };
     run_tiles(std::false_type{}, n_clean);
-    run_tiles(std::true_type{}, n_tiles);
+    run_tiles(std::true_type{}, t_hi);
     // the last tile's loads (of no page) are complete before the workgroup
     // can end and its LDS be handed on
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -590,6 +614,27 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
     for (int rb = 0; rb < RB; ++rb) {
       const float2 lh = swap_halves32(l[rb]);
       const float l_tot = lh.x + lh.y;
+      if constexpr (SPLIT) {
+        if (slot >= 0) {
+          if (!wave_rows) continue;
+          const int64_t blk =
+              ((int64_t)slot * p.hkv + h) * (C::ROWS / 32) + (RB * wave + rb);
+          const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+          float* po = p.partial_o + blk * (32 * D) + 4 * lane;
+#pragma unroll
+          for (int dt = 0; dt < C::DT; ++dt)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+              f32x4 w;
+#pragma unroll
+              for (int i = 0; i < 4; ++i) w[i] = o[rb][dt][4 * i4 + i] * inv;
+              *reinterpret_cast<f32x4*>(po + (4 * dt + i4) * 256) = w;
+            }
+          if (half == 0)
+            p.partial_lse[blk * 32 + col] = l_tot > 0.f ? m[rb] + log2f(l_tot) : -INFINITY;
+          continue;
+        }
+      }
       if (!rvalid[rb]) continue;
       const int row = 32 * (RB * wave + rb) + col;
       const int qi = q_lo + row / g;
@@ -629,20 +674,152 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
   body(std::false_type{}, stage0, stage1, wave, h);
 }
 
+// Merge of the cut tiles of a split plan:
+// o = sum_k 2^(lse_k - M) o_k / sum_k 2^(lse_k - M) over a row's pieces.
+// Unit: 32 rows x 32 d of one cut tile and KV head; a workgroup's four waves
+// take pieces w, w + 4, ... (kPieces loads of each lane at a time), and add
+// up through LDS in wave order.  Bound by the partials' bytes (P x 2 x 128 KiB
+// a tile and head, from the XCD's L2 or the Infinity Cache where they fit)
+// and, with few units, by the latency of the piece loop: hence the small
+// units.  Units run over the grid, with the KV head lowest as in
+// prefill_kernel, so a head's partials are read on the XCD that wrote them
+// (Hkv = 8).
+struct PrefillMergeArgs {
+  const PrefillMerge* merges;
+  const int32_t* n_merge;
+  int32_t cap, batch_size, hq, hkv, g, n_slots;
+  const int32_t* qo_indptr;
+  const float* po;
+  const float* pl;
+  uint16_t* out;
+  float* lse;
+};
+
+constexpr int kPrefillMergeWaves = 4;
+constexpr int kPrefillMergeGrid = 2048;  // workgroups: one resident set of waves
+
+template <bool BF16, int D>
+__global__ void __launch_bounds__(kWave * kPrefillMergeWaves)
+    prefill_merge_kernel(PrefillMergeArgs a) {
+  constexpr int DT = D / 32, BLKS = kPrefillRows / 32, NW = kPrefillMergeWaves;
+  constexpr int kPieces = 4;
+  __shared__ float s_m[NW][kWave], s_den[NW][kWave];
+  __shared__ f32x4 s_num[NW][4][kWave];
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const int n_merge = min(uniform(load_invariant(a.n_merge)), a.cap);
+  const int64_t units = (int64_t)n_merge * BLKS * DT * a.hkv;
+  for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
+    const int h = (int)(u % a.hkv);
+    const int v = (int)(u / a.hkv);
+    const int dt = v % DT, blk = v / DT % BLKS;
+    const int32_t* mp = reinterpret_cast<const int32_t*>(a.merges + v / (DT * BLKS));
+    const int b = uniform(load_invariant(mp + 0));
+    const int q_lo = uniform(load_invariant(mp + 1));
+    const int slot0 = uniform(load_invariant(mp + 3));
+    const int n = uniform(load_invariant(mp + 4));
+    // a merge list that does not match this launch is skipped, never followed
+    // (uniform over the workgroup, as every condition up to the barriers)
+    if (b < 0 || b >= a.batch_size || q_lo < 0 || slot0 < 0 || n < 1 || n > a.n_slots - slot0)
+      continue;
+    const int qo_start = uniform(load_invariant(a.qo_indptr + b));
+    const int q_hi = min(uniform(load_invariant(mp + 2)),
+                         uniform(load_invariant(a.qo_indptr + b + 1)) - qo_start);
+    if (32 * blk >= (q_hi - q_lo) * a.g) continue;
+    float M = -INFINITY, den = 0.f;
+    f32x4 num[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) num[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave; k0 < n; k0 += NW * kPieces) {
+      float lv[kPieces];
+      f32x4 ov[kPieces][4];
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j) {
+        const int k = k0 + NW * j;
+        lv[j] = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ov[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (k < n) {
+          const int64_t at = ((int64_t)(slot0 + k) * a.hkv + h) * BLKS + blk;
+          lv[j] = a.pl[at * 32 + col];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            ov[j][i] = *reinterpret_cast<const f32x4*>(a.po + at * (32 * D) +
+                                                       (4 * dt + i) * 256 + 4 * lane);
+        }
+      }
+      float Mb = M;
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j) Mb = fmaxf(Mb, lv[j]);
+      const float r = M == -INFINITY ? 0.f : exp2f(M - Mb);
+      den *= r;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) num[i] *= r;
+#pragma unroll
+      for (int j = 0; j < kPieces; ++j) {
+        const float wt = lv[j] == -INFINITY ? 0.f : exp2f(lv[j] - Mb);
+        den += wt;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) num[i][e] = fmaf(wt, ov[j][i][e], num[i][e]);
+      }
+      M = Mb;
+    }
+    s_m[wave][lane] = M;
+    s_den[wave][lane] = den;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_num[wave][i][lane] = num[i];
+    __syncthreads();
+    // wave i finishes register quad i: d = 32 dt + 8 i + 4 half + [0, 4)
+    M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][lane]);
+    den = 0.f;
+    f32x4 o4 = {0.f, 0.f, 0.f, 0.f};
+    if (M != -INFINITY) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float mw = s_m[w][lane];
+        const float wt = mw == -INFINITY ? 0.f : exp2f(mw - M);
+        den = fmaf(wt, s_den[w][lane], den);
+        const f32x4 x = s_num[w][wave][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o4[e] = fmaf(wt, x[e], o4[e]);
+      }
+      o4 *= 1.f / den;
+    }
+    const int row = 32 * blk + col;
+    const int qi = q_lo + row / a.g;
+    if (qi < q_hi) {
+      const int64_t orow = (int64_t)(qo_start + qi) * a.hq + h * a.g + row % a.g;
+      u32x2 w2;
+      w2[0] = pack2_16<BF16>(o4[0], o4[1]);
+      w2[1] = pack2_16<BF16>(o4[2], o4[3]);
+      *reinterpret_cast<u32x2*>(a.out + orow * D + 32 * dt + 8 * wave + 4 * half) = w2;
+      if (a.lse && dt == 0 && wave == 0 && half == 0)
+        a.lse[orow] = M != -INFINITY ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
+    }
+    __syncthreads();  // the sums are read before the next unit writes its own
+  }
+}
+
 using PrefillFn = void (*)(PrefillParams);
 
 template <int D, bool BF16, bool FP8>
-PrefillFn prefill_fn() {
-  return prefill_kernel<D, BF16, FP8, kPrefillRB>;
+PrefillFn prefill_fn(bool split) {
+  return split ? prefill_kernel<D, BF16, FP8, kPrefillRB, true>
+               : prefill_kernel<D, BF16, FP8, kPrefillRB, false>;
 }
 
-static PrefillFn pick_prefill(int d, bool bf16, bool fp8) {
+static PrefillFn pick_prefill(int d, bool bf16, bool fp8, bool split) {
   if (d == 64) {
-    if (bf16) return fp8 ? prefill_fn<64, true, true>() : prefill_fn<64, true, false>();
-    return fp8 ? prefill_fn<64, false, true>() : prefill_fn<64, false, false>();
+    if (bf16) return fp8 ? prefill_fn<64, true, true>(split) : prefill_fn<64, true, false>(split);
+    return fp8 ? prefill_fn<64, false, true>(split) : prefill_fn<64, false, false>(split);
   }
-  if (bf16) return fp8 ? prefill_fn<128, true, true>() : prefill_fn<128, true, false>();
-  return fp8 ? prefill_fn<128, false, true>() : prefill_fn<128, false, false>();
+  if (bf16) return fp8 ? prefill_fn<128, true, true>(split) : prefill_fn<128, true, false>(split);
+  return fp8 ? prefill_fn<128, false, true>(split) : prefill_fn<128, false, false>(split);
 }
 
 // ----------------------------------------------------------------------------
@@ -657,6 +834,9 @@ static PrefillFn pick_prefill(int d, bool bf16, bool fp8) {
 // tile's output is the same wherever it runs.  Entries past the tiles, up to
 // the plan's capacity, get b = -1 (the attention workgroups return at once);
 // tiles beyond the capacity are dropped and counted in `dropped`.
+// Plans with `slots` > 0 write PrefillPiece entries and cut long tiles of a
+// small step by the host planner's rule (plan.h): 8 threads count the pieces
+// of each of the 128 candidate cuts.
 struct PrefillPlanArgs {
   const int32_t* qo_indptr;
   const int32_t* kv_indptr;
@@ -664,6 +844,11 @@ struct PrefillPlanArgs {
   int32_t batch_size, q_tile, g, pair, cap;
   PrefillItem* items;
   int32_t* dropped;
+  // plans that may cut tiles: pieces per KV head, list entries
+  int32_t slots, entries;
+  PrefillPiece* pieces;
+  PrefillMerge* merges;
+  int32_t* n_merge;
 };
 
 constexpr int kPrefillPlanThreads = 1024;
@@ -674,6 +859,10 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
   __shared__ int start[kPrefillDevMaxBatch + 1];  // first tile of each sequence
   __shared__ int red[kPrefillPlanThreads / kWave];
   __shared__ long long key[kPrefillDevSortMax];
+  static_assert(kPrefillPlanThreads == 8 * kPrefillSplitMaxPieces, "8 threads per cut");
+  __shared__ int kv_tiles[kPrefillDevSortMax];  // KV tiles, then first entry, by list place
+  __shared__ int t_max_s;
+  __shared__ unsigned best_s;  // the best cut's P << 16 | pieces
   const int t = threadIdx.x;
   const int B = min(max(a.batch_size, 0), kPrefillDevMaxBatch);
   auto qo_len = [&](int b) {
@@ -719,7 +908,7 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
     const int qo = qo_len(b);
     const int q_lo = (i - start[b]) * a.q_tile;  // < qo
     const int q_hi = qo - q_lo > a.q_tile ? q_lo + a.q_tile : qo;
-    if (cost) {
+    if (cost) {  // kv tokens of the tile's last row
       const int np = max(a.kv_indptr[b + 1] - a.kv_indptr[b], 0);
       const int last = min(max(a.last_page_len[b], 1), kPage);
       const int64_t kv_len = np > 0 ? (int64_t)(np - 1) * kPage + last : 0;
@@ -728,49 +917,125 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
     const int flag = a.pair && (int64_t)(q_hi - q_lo) * a.g <= kPrefillRows / 2 ? 1 : -1;
     return PrefillItem{b, q_lo, q_hi, flag};
   };
+  auto put = [&](int at, const PrefillItem& it) {
+    if (a.slots > 0)
+      a.pieces[at] = PrefillPiece{it.b, it.q_lo, it.q_hi, it.slot, 0, 1, -1, 0};
+    else
+      a.items[at] = it;
+  };
+  int used = n_tiles;  // list entries written
+  int n_merge = 0;
   if (n_tiles <= kPrefillDevSortMax) {
     // one tile per thread; its rank among unique keys (cost, then sequence
     // order) is its place in the list
     PrefillItem it{-1, 0, 0, -1};
+    int rank = 0, mine_t = 0;
     if (t < n_tiles) {
       int64_t cost = 0;
       it = tile(t, &cost);
       key[t] = (cost << 10) | (kPrefillDevSortMax - 1 - t);
+      mine_t = (int)((cost + kPrefillKvTile - 1) / kPrefillKvTile);
+    }
+    if (t == 0) {
+      t_max_s = 0;
+      best_s = 0;
     }
     __syncthreads();
     if (t < n_tiles) {
       const long long mk = key[t];
-      int rank = 0;
       for (int j = 0; j < n_tiles; ++j) rank += key[j] > mk ? 1 : 0;
+      kv_tiles[rank] = mine_t;
+      if (rank == 0) t_max_s = mine_t;
+    }
+    __syncthreads();
+    // the cut, 0 for none (every condition is uniform)
+    int len = 0;
+    const int t_max = t_max_s;
+    if (n_tiles <= a.slots && t_max >= 2 * kPrefillSplitMinTiles && total <= a.cap) {
+      const int P = 1 + (t >> 3);
+      const int lp = (t_max + P - 1) / P;
+      int count = 0;
+      for (int j = t & 7; j < n_tiles; j += 8) {
+        const int x = kv_tiles[j];
+        count += x > 0 ? (x + lp - 1) / lp : 1;
+      }
+#pragma unroll
+      for (int off = 1; off < 8; off <<= 1) count += __shfl_xor(count, off);
+      if (P > 1 && lp >= kPrefillSplitMinTiles && count <= a.slots && (t & 7) == 0)
+        atomicMax(&best_s, (unsigned)P << 16 | (unsigned)count);
+      __syncthreads();
+      const int best = (int)(best_s >> 16);
+      if (best > 1) {
+        const int lb = (t_max + best - 1) / best;
+        if (prefill_split_pays(t_max, lb, (int)(best_s & 0xffff), a.slots)) len = lb;
+      }
+    }
+    if (len > 0) {
+      // thread r takes list place r: pieces and cut tiles before it
+      const int x = t < n_tiles ? kv_tiles[t] : 0;
+      const int np = t < n_tiles ? (x > 0 ? (x + len - 1) / len : 1) : 0;
+      int all = 0, cut = 0;
+      const int first = block_excl_scan<kPrefillPlanThreads>(np, &all, red);
+      const int m_at = block_excl_scan<kPrefillPlanThreads>(np > 1 ? 1 : 0, &cut, red);
+      used = all;
+      n_merge = cut;
+      // the place's pieces and merge entry, packed for the tile's own thread
+      if (t < n_tiles) {
+        kv_tiles[t] = first;
+        key[t] = ((long long)np << 32) | (long long)m_at;
+      }
+      __syncthreads();
+      if (t < n_tiles) {
+        const int at = kv_tiles[rank];
+        const int n = (int)(key[rank] >> 32);
+        for (int k = 0; k < n; ++k)
+          a.pieces[at + k] =
+              PrefillPiece{it.b, it.q_lo, it.q_hi, -1, k, n, n > 1 ? at + k : -1, 0};
+        if (n > 1)
+          a.merges[(int)(key[rank] & 0x7fffffff)] =
+              PrefillMerge{it.b, it.q_lo, it.q_hi, at, n, 0, 0, 0};
+      }
+    } else if (t < n_tiles) {
       // paired tiles alternate between the even and the odd head of a head
       // pair by list position, so both XCDs of the pair share them
       if (it.slot > 0) it.slot = 1 + (rank & 1);
-      a.items[rank] = it;
+      put(rank, it);
     }
   } else {
     for (int i = t; i < n_tiles; i += kPrefillPlanThreads) {
       PrefillItem it = tile(i, nullptr);
       if (it.slot > 0) it.slot = 1 + (i & 1);
-      a.items[i] = it;
+      put(i, it);
     }
   }
-  for (int i = n_tiles + t; i < a.cap; i += kPrefillPlanThreads)
-    a.items[i] = PrefillItem{-1, 0, 0, -1};
+  if (a.slots > 0 && t == 0) *a.n_merge = n_merge;
+  const int end = a.slots > 0 ? a.entries : a.cap;
+  for (int i = used + t; i < end; i += kPrefillPlanThreads) put(i, PrefillItem{-1, 0, 0, -1});
 }
 
 }  // namespace pa
 
 namespace pa {
 
+// The cut tiles' count of a split plan's merge list.
+static int32_t* split_count(const pagedattn_plan* plan) {
+  return reinterpret_cast<int32_t*>(static_cast<char*>(plan->workspace) + kWsHeader);
+}
+
 // The q-tile list of a device prefill plan, cut from the metadata on the
 // device by one workgroup (prefill_plan_kernel) on `stream`.
 static int launch_prefill_plan(const pagedattn_plan* plan, const int32_t* qo_indptr,
                                const int32_t* kv_indptr, const int32_t* kv_last_page_len,
                                void* stream, const char* who) {
+  const bool split = plan->prefill_split;
   PrefillPlanArgs a{qo_indptr, kv_indptr, kv_last_page_len, plan->batch_size,
                     plan->q_tile, plan->hq / plan->hkv, plan->prefill_pair ? 1 : 0,
-                    plan->n_items, static_cast<PrefillItem*>(plan->items_dev),
-                    reinterpret_cast<int32_t*>(static_cast<char*>(plan->workspace) + 12)};
+                    split ? plan->q_cap : plan->n_items,
+                    static_cast<PrefillItem*>(plan->items_dev),
+                    reinterpret_cast<int32_t*>(static_cast<char*>(plan->workspace) + 12),
+                    split ? plan->n_slots : 0, plan->n_items,
+                    static_cast<PrefillPiece*>(plan->items_dev),
+                    static_cast<PrefillMerge*>(plan->merge_dev), split_count(plan)};
   hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPrefillPlanThreads), 0,
                      (hipStream_t)stream, a);
   return check_launch(who);
@@ -850,7 +1115,7 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   if (num_pages < 0 || num_indices < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: negative sizes", who);
   PrefillParams p;
-  p.items = static_cast<const PrefillItem*>(plan->items_dev);
+  p.items = plan->items_dev;
   p.n_items = plan->n_items;
   p.batch_size = plan->batch_size;
   p.q = static_cast<const uint16_t*>(q);
@@ -871,7 +1136,11 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   p.g = plan->hq / plan->hkv;
   p.causal = causal ? 1 : 0;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
-  PrefillFn fn = pick_prefill(plan->d, q_dtype == PAGEDATTN_BF16, fp8);
+  p.partial_o = plan->partial_o;
+  p.partial_lse = plan->partial_lse;
+  p.n_slots = plan->n_slots;
+  const bool bf16 = q_dtype == PAGEDATTN_BF16;
+  PrefillFn fn = pick_prefill(plan->d, bf16, fp8, plan->prefill_split);
   if (plan->implicit && !plan->dev_table) {
     // the work list of this run, built on the device ahead of the attention
     // (unless pagedattn_prefill_plan_device_update built it for the step)
@@ -880,7 +1149,21 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   }
   hipLaunchKernelGGL(fn, dim3(plan->n_items * plan->hkv), dim3(64 * kPrefillWaves), 0,
                      (hipStream_t)stream, p);
-  return check_launch(who);
+  const int rc = check_launch(who);
+  if (rc || !plan->prefill_split) return rc;
+  // host plans know their cut tiles; a device plan's are at most half its
+  // slots, and its merge workgroups find out how many there are
+  const int cap = plan->implicit ? plan->n_slots / 2 : plan->n_merge;
+  PrefillMergeArgs m{static_cast<const PrefillMerge*>(plan->merge_dev), split_count(plan), cap,
+                     plan->batch_size, plan->hq, plan->hkv, p.g, plan->n_slots, qo_indptr,
+                     plan->partial_o, plan->partial_lse, p.out, lse};
+  const int64_t units = (int64_t)cap * (kPrefillRows / 32) * (plan->d / 32) * plan->hkv;
+  auto* mfn = plan->d == 64
+                  ? (bf16 ? prefill_merge_kernel<true, 64> : prefill_merge_kernel<false, 64>)
+                  : (bf16 ? prefill_merge_kernel<true, 128> : prefill_merge_kernel<false, 128>);
+  hipLaunchKernelGGL(mfn, dim3((unsigned)std::min<int64_t>(units, kPrefillMergeGrid)),
+                     dim3(kWave * kPrefillMergeWaves), 0, (hipStream_t)stream, m);
+  return check_launch("prefill_run(merge)");
 }
 
 }  // extern "C"

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdlib>
+#include <cstring>
 #include <vector>
 
 #include "plan_internal.h"
@@ -20,6 +21,54 @@ namespace pa {
 static bool prefill_pairing() {
   const char* env = std::getenv("PAGEDATTN_PREFILL_PAIR");
   return !(env && std::atoi(env) == 0);
+}
+
+// Split-KV prefill (plan.h) is planned by default; PAGEDATTN_PREFILL_SPLIT=0
+// keeps every q-tile whole.
+static bool prefill_splitting() {
+  const char* env = std::getenv("PAGEDATTN_PREFILL_SPLIT");
+  return !(env && std::atoi(env) == 0);
+}
+
+// Pieces per KV head: one workgroup per CU.  (At D = 64 a CU holds two, but
+// they share its matrix cores: cutting for 512 workgroups ran a 4 x 512-token
+// TinyLlama step over 1000-token prefixes in 47 us, uncut 35 us.)
+static int64_t prefill_split_slots(int hkv) {
+  int cus = device_cu_count();
+  if (cus <= 0) cus = 256;
+  return std::max(1, cus / hkv);
+}
+
+// KV tiles per piece of the q-tiles with `tiles` KV tiles (the rule in
+// plan.h; prefill_plan_kernel applies the same one), or 0 to keep them whole.
+static int prefill_piece_tiles(const std::vector<int>& tiles, int64_t slots) {
+  if (tiles.empty() || (int64_t)tiles.size() > slots) return 0;
+  const int t_max = *std::max_element(tiles.begin(), tiles.end());
+  auto len = [&](int p) { return (t_max + p - 1) / p; };
+  auto count = [&](int p) {
+    int64_t n = 0;
+    for (int t : tiles) n += t > 0 ? (t + len(p) - 1) / len(p) : 1;
+    return n;
+  };
+  auto fits = [&](int p) { return len(p) >= kPrefillSplitMinTiles && count(p) <= slots; };
+  int lo = 1, hi = kPrefillSplitMaxPieces;  // more pieces only ever take more slots
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (t_max > 0 && fits(mid)) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo > 1 && prefill_split_pays(t_max, len(lo), count(lo), slots) ? len(lo) : 0;
+}
+
+// The device side of a split plan: work list, merge list and partials.
+static void set_split(pagedattn_plan* plan, const PrefillSplitLayout& lay, int64_t slots) {
+  char* ws = static_cast<char*>(plan->workspace);
+  plan->prefill_split = true;
+  plan->n_slots = (int)slots;
+  plan->items_dev = ws + lay.off_pieces;
+  plan->merge_dev = ws + lay.off_merges;
+  plan->partial_o = reinterpret_cast<float*>(ws + lay.off_po);
+  plan->partial_lse = reinterpret_cast<float*>(ws + lay.off_pl);
 }
 
 }  // namespace pa
@@ -73,6 +122,20 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
     return set_error(PAGEDATTN_ERR_WORKSPACE,
                      "%s: %lld q-tiles do not fit the %zu-byte workspace", who,
                      (long long)n_tiles, workspace_bytes);
+  auto finish = [&](pagedattn_plan* pl) {
+    pl->batch_size = batch_size;
+    pl->hq = num_qo_heads;
+    pl->hkv = num_kv_heads;
+    pl->d = head_dim;
+    pl->page_size = page_size;
+    pl->q_tile = q_tile;
+    pl->total_qo =
+        batch_size > 0 ? (int64_t)qo_indptr_host[batch_size] - qo_indptr_host[0] : 0;
+    pl->implicit = false;
+    pl->shared = false;
+    pl->dev_table = false;
+    pl->mode = kPlanPrefill;
+  };
   std::vector<PrefillItem> items;
   std::vector<int64_t> cost;
   items.reserve((size_t)n_tiles);
@@ -95,6 +158,46 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(),
                    [&](int a, int c) { return cost[a] > cost[c]; });
+  plan->prefill_split = false;
+  const int64_t slots = prefill_split_slots(num_kv_heads);
+  const PrefillSplitLayout lay = prefill_split_layout(slots, slots, num_kv_heads, head_dim);
+  int piece_tiles = 0;
+  if (prefill_splitting() && lay.end <= workspace_bytes && (int64_t)items.size() <= slots) {
+    std::vector<int> tiles;
+    for (int64_t c : cost) tiles.push_back((int)((c + kPrefillKvTile - 1) / kPrefillKvTile));
+    piece_tiles = prefill_piece_tiles(tiles, slots);
+  }
+  if (piece_tiles > 0) {
+    std::vector<PrefillPiece> pieces;
+    std::vector<PrefillMerge> merges;
+    for (int i : order) {
+      const PrefillItem& it = items[i];
+      const int t = (int)((cost[i] + kPrefillKvTile - 1) / kPrefillKvTile);
+      const int n = std::max(1, (t + piece_tiles - 1) / piece_tiles);
+      const int at = (int)pieces.size();
+      for (int k = 0; k < n; ++k)
+        pieces.push_back(PrefillPiece{it.b, it.q_lo, it.q_hi, -1, k, n, n > 1 ? at + k : -1, 0});
+      if (n > 1) merges.push_back(PrefillMerge{it.b, it.q_lo, it.q_hi, at, n, 0, 0, 0});
+    }
+    const size_t host_bytes = lay.off_po - kWsHeader;
+    plan->host.assign(host_bytes / sizeof(int32_t), 0);
+    char* hb = reinterpret_cast<char*>(plan->host.data());
+    const int32_t n_merge = (int32_t)merges.size();
+    std::memcpy(hb + (lay.off_count - kWsHeader), &n_merge, sizeof(n_merge));
+    std::memcpy(hb + (lay.off_pieces - kWsHeader), pieces.data(),
+                sizeof(PrefillPiece) * pieces.size());
+    std::memcpy(hb + (lay.off_merges - kWsHeader), merges.data(),
+                sizeof(PrefillMerge) * merges.size());
+    plan->workspace = workspace;
+    plan->workspace_bytes = workspace_bytes;
+    rc = upload_plan(plan, who, host_bytes, lay.end, stream);
+    if (rc) return rc;
+    plan->n_items = (int)pieces.size();
+    plan->n_merge = n_merge;
+    set_split(plan, lay, slots);
+    finish(plan);
+    return PAGEDATTN_OK;
+  }
   const size_t host_bytes = sizeof(PrefillItem) * items.size();
   plan->host.assign((host_bytes + 3) / 4, 0);
   auto* dst = reinterpret_cast<PrefillItem*>(plan->host.data());
@@ -110,22 +213,11 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
   rc = upload_plan(plan, who, host_bytes, ws_align(kWsHeader + host_bytes),
                    stream);
   if (rc) return rc;
-  plan->batch_size = batch_size;
-  plan->hq = num_qo_heads;
-  plan->hkv = num_kv_heads;
-  plan->d = head_dim;
-  plan->page_size = page_size;
   plan->n_items = (int)items.size();
   plan->n_merge = 0;
   plan->n_slots = 0;
-  plan->q_tile = q_tile;
-  plan->total_qo =
-      batch_size > 0 ? (int64_t)qo_indptr_host[batch_size] - qo_indptr_host[0] : 0;
   plan->items_dev = static_cast<char*>(workspace) + kWsHeader;
-  plan->implicit = false;
-  plan->shared = false;
-  plan->dev_table = false;
-  plan->mode = kPlanPrefill;
+  finish(plan);
   return PAGEDATTN_OK;
 }
 
@@ -174,6 +266,18 @@ int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,
   plan->q_tile = q_tile;
   plan->total_qo = max_qo_tokens;
   plan->items_dev = static_cast<char*>(workspace) + kWsHeader;
+  // a plan whose workspace holds the partials may cut tiles, on the host
+  // plan's rule (the tiles are known to the plan kernel only)
+  plan->prefill_split = false;
+  const int64_t slots = prefill_split_slots(num_kv_heads);
+  const int64_t entries = std::max(cap, slots);
+  const PrefillSplitLayout lay = prefill_split_layout(entries, slots, num_kv_heads, head_dim);
+  if (prefill_splitting() && slots >= 2 && slots <= kPrefillDevSortMax &&
+      lay.end <= workspace_bytes && entries * num_kv_heads <= INT32_MAX) {
+    plan->n_items = (int)entries;
+    plan->q_cap = (int)cap;
+    set_split(plan, lay, slots);
+  }
   plan->mode = kPlanPrefill;
   return PAGEDATTN_OK;
 }

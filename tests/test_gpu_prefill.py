@@ -178,3 +178,37 @@ def test_prefill_paired_tiles_bit_identical(gpu, monkeypatch, case, causal):
     out0, lse0 = run_prefill(gpu, meta, pool, q, hq, hkv, d, causal=causal)
     assert torch.equal(out0, out1)
     assert torch.equal(lse0, lse1)
+
+
+# (cached prefix, new chunk) of steps with few q-tiles over long prefixes: the
+# KV tiles are cut into pieces (one sequence of one token up to ragged batches
+# with short, empty-prefix and causal-diagonal tiles among the long ones)
+SPLIT_STEPS = {"one_token": [(5000, 1)], "ragged": [(3000, 70), (0, 5), (1500, 33), (64, 7)],
+               "chunk": [(2011, 150)], "diagonal": [(0, 900)]}
+
+
+@pytest.mark.parametrize("step", sorted(SPLIT_STEPS))
+@pytest.mark.parametrize("d,hq,hkv,fp8", [(128, 32, 8, False), (64, 32, 4, False),
+                                          (128, 8, 1, False), (128, 12, 3, True),
+                                          (64, 32, 4, True)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_split_kv(gpu, monkeypatch, step, d, hq, hkv, fp8, causal):
+    monkeypatch.delenv("PAGEDATTN_PREFILL_SPLIT", raising=False)
+    computed = [c for c, _ in SPLIT_STEPS[step]]
+    chunks = [n for _, n in SPLIT_STEPS[step]]
+    meta, pool, q = prefill_case(gpu, computed, chunks, hq, hkv, d, seed=d + hkv)
+    scales = None
+    if fp8:
+        pool, scales = pagedattn.quantize_pages_e4m3(pool)
+    ref_o, ref_l = oracle_prefill(meta, pool, q, causal=causal, scales=scales)
+    out, lse = run_prefill(gpu, meta, pool, q, hq, hkv, d, causal=causal, kv_scales=scales)
+    tol = TOL_FP8 if fp8 else TOL_BF16
+    assert max_err(out, ref_o) <= tol
+    assert lse_err(lse, ref_l) <= TOL_LSE
+    # a workspace without room for the partials keeps the tiles whole
+    small = torch.zeros(1 << 16, dtype=torch.uint8, device=gpu)
+    out_w, lse_w = run_prefill(gpu, meta, pool, q, hq, hkv, d, causal=causal, kv_scales=scales,
+                               ws=small)
+    assert not torch.equal(lse, lse_w)  # the large workspace's plan was cut
+    assert max_err(out_w, ref_o) <= tol
+    assert lse_err(lse_w, ref_l) <= TOL_LSE

@@ -263,3 +263,51 @@ def test_chunked_prefill_step_graph_replay(gpu, table):
         rows = list(range(q0 + lo, q0 + n))
         assert max_err(eager.out[rows], ref_o) <= TOL_BF16, b
         assert lse_err(eager.lse[rows], ref_l) <= TOL_LSE, b
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(128, 32, 8), (64, 32, 4), (128, 12, 3)])
+def test_prefill_device_plan_cuts_kv_like_the_host_plan(gpu, d, hq, hkv):
+    """Steps whose KV ranges are cut, steps kept whole and an empty one, one
+    after the other through one captured graph and an eager device plan: both
+    give the host plan's bits (the capacity leaves list entries unused)."""
+    steps = [[(5000, 1), (40, 20)], [(0, 30), (16, 2)], [(0, 0), (0, 0)],
+             [(2000, 33), (3000, 64)], [(0, 20), (900, 5)], [(1200, 60), (7, 0)]]
+    bsz, tokens, maxp = 2, 100, 320
+    rng = np.random.default_rng(d + hkv)
+    tables, num_pages = random_tables(rng, [16 * maxp] * bsz, extra_pages=2)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(d)
+    pool = torch.randn((num_pages, 2, hkv, 16, d), generator=g, device=gpu).to(torch.bfloat16)
+    q = torch.randn((tokens, hq, d), generator=g, device=gpu).to(torch.bfloat16)
+    qo, kv = (torch.zeros(bsz + 1, dtype=torch.int32, device=gpu) for _ in range(2))
+    ind = torch.zeros(bsz * maxp, dtype=torch.int32, device=gpu)
+    last = torch.ones(bsz, dtype=torch.int32, device=gpu)
+    out = torch.zeros_like(q)
+    lse = torch.zeros((tokens, hq), dtype=torch.float32, device=gpu)
+    w = pagedattn.BatchPrefillWithPagedKVCacheWrapper(workspace(gpu), "HND")
+    w.plan(qo, kv, ind, last, hq, hkv, d, 16, causal=True, q_data_type=torch.bfloat16,
+           device_plan=True, max_qo_tokens=tokens)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        w.run(q, pool, out=out, lse=lse)
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    cg = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(cg):
+        w.run(q, pool, out=out, lse=lse)
+    for i, step in enumerate(steps):
+        meta = prefill_metadata([t[:-(-(c + n) // 16)] for t, (c, n) in zip(tables, step)],
+                                [c for c, _ in step], [n for _, n in step])
+        qo.copy_(i32(meta.qo_indptr, gpu))
+        kv.copy_(i32(meta.kv_indptr, gpu))
+        ind[:len(meta.kv_indices)] = i32(meta.kv_indices, gpu)
+        last.copy_(i32(meta.kv_last_page_len, gpu))
+        n = meta.nnz
+        cg.replay()
+        got = out.clone(), lse.clone()
+        eager = w.run(q, pool, return_lse=True)
+        torch.cuda.synchronize()
+        o_h, l_h, _ = _prefill(gpu, meta, pool, q[:n], hq, hkv, d, device_plan=False)
+        for o, l in (got, eager):
+            assert torch.equal(o[:n], o_h) and torch.equal(l[:n], l_h), i
