@@ -10,12 +10,15 @@ point raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
 
 LIB_NAME = "libpagedattn.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
+CALLS_PATH = os.path.join(os.path.dirname(LIB_PATH), "_calls.so")
 
 # element type codes (include/pagedattn.h)
 F16, BF16, E4M3, F32 = 0, 1, 2, 3
@@ -148,12 +151,41 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_calls = None
+
+
+def calls():
+    """The extension module of the per-layer calls (csrc/calls.cpp), loaded
+    once and bound to the library's entry points; raises if it is not built."""
+    global _calls
+    if _calls is None:
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(
+                f"{CALLS_PATH} is not built; run __graft_entry__.build() or "
+                "`make -C llm-inference-runtime_amd/csrc`")
+        name = __package__ + "._calls"
+        loader = importlib.machinery.ExtensionFileLoader(name, CALLS_PATH)
+        mod = importlib.util.module_from_spec(
+            importlib.util.spec_from_file_location(name, CALLS_PATH, loader=loader))
+        loader.exec_module(mod)
+        handle = lib()
+        mod.bind(torch._C._cuda_getCurrentRawStream,
+                 {n: ctypes.cast(getattr(handle, n), ctypes.c_void_p).value for n in EXPORTED})
+        _calls = mod
+    return _calls
+
+
+def raise_status(name: str, rc: int) -> None:
+    """Raise PagedAttnError for entry point `name`'s non-zero status."""
+    msg = lib().pagedattn_last_error()
+    raise PagedAttnError(name, rc, msg.decode() if msg else "")
+
+
 def call(name: str, *args) -> None:
     """Call entry point `name`; raise PagedAttnError on a non-zero status."""
     rc = getattr(lib(), name)(*args)
     if rc != 0:
-        msg = lib().pagedattn_last_error()
-        raise PagedAttnError(name, rc, msg.decode() if msg else "")
+        raise_status(name, rc)
 
 
 def dtype_code(dt: torch.dtype) -> int:

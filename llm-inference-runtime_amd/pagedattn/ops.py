@@ -104,6 +104,16 @@ def _check_scales(kv_scales, paged_kv_cache) -> torch.Tensor | None:
     return kv_scales.contiguous()
 
 
+def _native(fn: str, entry: str, *args):
+    """One per-layer call through csrc/calls.cpp: its result, or
+    NotImplemented where the arguments need the general path below it (which
+    converts them or raises)."""
+    r = getattr(_lib._calls or _lib.calls(), fn)(*args)
+    if type(r) is int:
+        _lib.raise_status(entry, r)
+    return r
+
+
 def _check_rows(x: torch.Tensor, name: str, heads: int | None, d: int | None):
     _require_cuda(x, name)
     if x.dim() != 3:
@@ -181,6 +191,11 @@ def append_paged_kv_cache(append_key: torch.Tensor, append_value: torch.Tensor,
     error_flag[1] is incremented once per 8-element piece of a written row
     that was clamped or had a bad scale.  Zeros mean every token landed
     intact."""
+    if kv_layout == "HND" and _native(
+            "append", "pagedattn_append_paged_kv_cache", append_key, append_value, batch_indices,
+            positions, paged_kv_cache, kv_indices, kv_indptr, kv_scales, error_flag,
+            kv_last_page_len) is None:
+        return
     num_pages, hkv, d = _check_pool(paged_kv_cache, None, None, kv_layout)
     _check_rows(append_key, "append_key", hkv, d)
     _check_rows(append_value, "append_value", hkv, d)
@@ -220,6 +235,11 @@ def rope_append_paged_kv_cache(q: torch.Tensor, append_key: torch.Tensor,
     (src/models/llama.py:175-210): q and append_key are rotated in place, the
     rotated K rows and the V rows land in their pages.  Same results as the
     two calls."""
+    if kv_layout == "HND" and _native(
+            "rope_append", "pagedattn_rope_append_paged_kv_cache", append_key, append_value,
+            batch_indices, positions, paged_kv_cache, kv_indices, kv_indptr, kv_scales,
+            error_flag, q, rope_scale, rope_theta) is None:
+        return
     num_pages, hkv, d = _check_pool(paged_kv_cache, None, None, kv_layout)
     _check_rows(q, "q", None, d)
     _check_rows(append_key, "append_key", hkv, d)
@@ -267,6 +287,11 @@ def append_paged_kv_cache_e4m3_amax(append_key: torch.Tensor, append_value: torc
     e4m3's normal range).  kv_scales [num_pages, 2, Hkv] is updated in place.
     Two sequences writing one page in the same call race: fork shared pages
     first (fork_pages)."""
+    if kv_layout == "HND" and _native(
+            "append_amax", "pagedattn_append_paged_kv_cache_e4m3_amax", append_key, append_value,
+            batch_indices, positions, paged_kv_cache, kv_indices, kv_indptr, kv_scales,
+            error_flag) is None:
+        return
     num_pages, hkv, d = _check_pool(paged_kv_cache, None, None, kv_layout)
     if paged_kv_cache.dtype != torch.float8_e4m3fn:
         raise ValueError("append_paged_kv_cache_e4m3_amax needs an e4m3 pool")
@@ -693,6 +718,17 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
         kernel (q and append_key themselves are left unrotated)."""
         if not self._planned:
             raise RuntimeError("plan()/begin_forward() must be called before run()/forward()")
+        scale = sm_scale if sm_scale is not None else self._sm_scale
+        if scale is None:
+            scale = 1.0 / math.sqrt(self._d)
+        entry = ("pagedattn_decode_run" if append_key is None else
+                 "pagedattn_decode_run_append" if rope is None else
+                 "pagedattn_decode_run_rope_append")
+        r = _native("decode_run", entry, self._plan.handle, q, paged_kv_cache, self._indices,
+                    self._indptr, self._last, self._bsz, self._hq, self._hkv, self._d, kv_scales,
+                    out, lse, return_lse, scale, append_key, append_value, rope, positions)
+        if r is not NotImplemented:
+            return r
         num_pages, _, _ = _check_pool(paged_kv_cache, self._hkv, self._d, self._kv_layout)
         _check_rows(q, "q", self._hq, self._d)
         if q.shape[0] != self._bsz:
@@ -706,9 +742,6 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
             raise ValueError("out must be a contiguous [batch, num_qo_heads, head_dim] tensor")
         if return_lse and lse is None:
             lse = torch.empty((self._bsz, self._hq), dtype=torch.float32, device=q.device)
-        scale = sm_scale if sm_scale is not None else self._sm_scale
-        if scale is None:
-            scale = 1.0 / math.sqrt(self._d)
         common = (ptr(paged_kv_cache), dtype_code(paged_kv_cache.dtype), ptr(scales),
                   num_pages, ptr(self._indices), self._indices.numel(), ptr(self._indptr),
                   ptr(self._last), ptr(out), ptr(lse), float(scale), _stream(q.device))
@@ -869,6 +902,16 @@ class BatchPrefillWithPagedKVCacheWrapper(_WrapperBase):
             causal: bool | None = None, sm_scale: float | None = None):
         if not self._planned:
             raise RuntimeError("plan()/begin_forward() must be called before run()/forward()")
+        scale = sm_scale if sm_scale is not None else self._sm_scale
+        if scale is None:
+            scale = 1.0 / math.sqrt(self._d)
+        is_causal = self._causal if causal is None else bool(causal)
+        r = _native("prefill_run", "pagedattn_prefill_run", self._plan.handle, q, paged_kv_cache,
+                    self._qo_indptr, self._indices, self._indptr, self._last, self._bsz,
+                    -1 if self._qo_rows is None else self._qo_rows, self._hq, self._hkv, self._d,
+                    kv_scales, out, lse, return_lse, is_causal, scale)
+        if r is not NotImplemented:
+            return r
         num_pages, _, _ = _check_pool(paged_kv_cache, self._hkv, self._d, self._kv_layout)
         _check_rows(q, "q", self._hq, self._d)
         if self._qo_rows is not None and q.shape[0] < self._qo_rows:
@@ -883,10 +926,6 @@ class BatchPrefillWithPagedKVCacheWrapper(_WrapperBase):
             raise ValueError("out must be a contiguous [nnz, num_qo_heads, head_dim] tensor")
         if return_lse and lse is None:
             lse = torch.empty((n, self._hq), dtype=torch.float32, device=q.device)
-        scale = sm_scale if sm_scale is not None else self._sm_scale
-        if scale is None:
-            scale = 1.0 / math.sqrt(self._d)
-        is_causal = self._causal if causal is None else bool(causal)
         call("pagedattn_prefill_run", self._plan.handle, ptr(q), q.stride(0), q.stride(1),
              dtype_code(q.dtype), ptr(self._qo_indptr), ptr(paged_kv_cache),
              dtype_code(paged_kv_cache.dtype), ptr(scales), num_pages, ptr(self._indices),

@@ -284,3 +284,68 @@ def test_rope_append_shapes_equal_separate(gpu, d, hq, hkv, nnz):
     torch.cuda.synchronize()
     assert torch.equal(a, b)
     assert torch.equal(pool_a, pool_b)
+
+
+@pytest.mark.parametrize("dtype,fp8", [(torch.bfloat16, False), (torch.float16, False),
+                                       (torch.bfloat16, True)])
+def test_native_calls_equal_the_general_path(gpu, monkeypatch, dtype, fp8):
+    # every per-layer call through the extension and, with it switched off,
+    # through the general path: same bits; int64 metadata goes the general way
+    hq, hkv, d = 8, 2, 64
+    g = torch.Generator(device=gpu)
+    g.manual_seed(3)
+    meta = prefill_metadata([[3, 1], [0, 4, 2]], [10, 20], [9, 20])
+    pool0 = torch.randn((6, 2, hkv, 16, d), generator=g, device=gpu).to(dtype)
+    scales0 = None
+    if fp8:
+        pool0, scales0 = pagedattn.quantize_pages_e4m3(pool0)
+        scales0 = torch.exp2(torch.ceil(torch.log2(scales0)))
+    qkv0 = torch.randn((meta.nnz, (hq + 2 * hkv) * d), generator=g, device=gpu).to(dtype)
+    ind, indptr = i32(meta.kv_indices, gpu), i32(meta.kv_indptr, gpu)
+    last, qo = i32(meta.kv_last_page_len, gpu), i32(meta.qo_indptr, gpu)
+    bi, pos = i32(meta.batch_indices, gpu), i32(meta.positions, gpu)
+    ws = torch.zeros(1 << 24, dtype=torch.uint8, device=gpu)
+
+    def step(cast):
+        pool, qkv = pool0.clone(), qkv0.clone()
+        scales = None if scales0 is None else scales0.clone()
+        q, k, v = (x.view(meta.nnz, -1, d) for x in
+                   qkv.split([hq * d, hkv * d, hkv * d], dim=-1))
+        flag = torch.zeros(2, dtype=torch.int32, device=gpu)
+        m = (cast(bi), cast(pos), pool, cast(ind), cast(indptr), last)
+        res = []
+        pagedattn.append_paged_kv_cache(k, v, *m, kv_layout="HND", kv_scales=scales,
+                                        error_flag=flag)
+        res += [pool.clone(), flag.clone()]
+        pagedattn.rope_append_paged_kv_cache(q, k, v, *m, kv_layout="HND", kv_scales=scales,
+                                             rope_theta=5e5)
+        res += [pool.clone(), qkv.clone()]
+        if fp8:
+            pagedattn.append_paged_kv_cache_e4m3_amax(k, v, *m, scales, kv_layout="HND")
+            res += [pool.clone(), scales.clone()]
+        pw = pagedattn.BatchPrefillWithPagedKVCacheWrapper(ws, "HND")
+        pw.plan(qo, indptr, ind, last, hq, hkv, d, 16, causal=True, q_data_type=dtype)
+        res += [pw.run(q, pool, kv_scales=scales)]
+        res += list(pw.run(q, pool, kv_scales=scales, causal=False, sm_scale=0.2,
+                           out=torch.empty_like(res[-1]), return_lse=True))
+        dw = pagedattn.BatchDecodeWithPagedKVCacheWrapper(ws, "HND")
+        dw.plan(indptr, ind, last, hq, hkv, d, 16, q_data_type=dtype)
+        q2, k2, v2 = (x[:2] for x in (q, k, v))
+        lse = torch.empty((2, hq), device=gpu)
+        res += [dw.run(q2, pool, kv_scales=scales)]
+        res += list(dw.run(q2, pool, kv_scales=scales, lse=lse, return_lse=True))
+        assert res[-1] is lse
+        res += [dw.run(q2, pool, kv_scales=scales, append_key=k2, append_value=v2)]
+        res += [dw.run(q2, pool, kv_scales=scales, append_key=k2, append_value=v2,
+                       rope=(1.0, 5e5), positions=cast(last * 0 + 17)), pool]
+        torch.cuda.synchronize()
+        return res
+
+    want = step(lambda t: t)
+    wide = step(lambda t: t.long())
+    monkeypatch.setattr(pagedattn.ops, "_native", lambda *a: NotImplemented)
+    general = step(lambda t: t)
+    for x, y, z in zip(want, wide, general):
+        x, y, z = (t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t
+                   for t in (x, y, z))
+        assert torch.equal(x, y) and torch.equal(x, z)

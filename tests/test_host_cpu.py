@@ -233,3 +233,27 @@ def test_cow_fork_decisions(monkeypatch):
         p = a2.allocate(1)
         a2.ref_counts[p[0]] = 2
         cow.fork_for_append(a2, [p], [5], None)
+
+
+def test_native_calls_leave_other_forms_to_the_general_path():
+    # anything but plain device tensors (here: host tensors, None, numbers) is
+    # handed back, for the general path to convert or refuse
+    calls = _lib.calls()
+    t = torch.zeros(2, 4, 64, dtype=torch.bfloat16)
+    i = torch.zeros(3, dtype=torch.int32)
+    pool = torch.zeros(4, 2, 4, 16, 64, dtype=torch.bfloat16)
+    for x in (t, None, 3, "x", torch.nn.Parameter(t)):
+        assert calls.decode_run(0, x, pool, i, i, i, 2, 4, 4, 64, None, None, None, False, 1.0,
+                                None, None, None, None) is NotImplemented
+        assert calls.prefill_run(0, x, pool, i, i, i, i, 2, 2, 4, 4, 64, None, None, None, False,
+                                 True, 1.0) is NotImplemented
+        assert calls.append(x, t, i, i, pool, i, i, None, None, i) is NotImplemented
+        assert calls.rope_append(x, t, i, i, pool, i, i, None, None, t, 1.0, 1e4) is NotImplemented
+        assert calls.append_amax(t, t, i, i, x, i, i, None, None) is NotImplemented
+    with pytest.raises(TypeError):
+        calls.append(t)
+    with pytest.raises(TypeError):
+        calls.prefill_run(0, t, pool, i, i, i, i, 2, 2, 4, 4, 64, None, None, None, False, True,
+                          "scale")
+    with pytest.raises(ValueError):
+        pagedattn.append_paged_kv_cache(t, t, i, i, pool, i, i, i, kv_layout="HND")
