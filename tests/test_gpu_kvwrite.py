@@ -76,6 +76,33 @@ def test_amax_append_prefill_then_decode(gpu, src, d):
     assert np.array_equal(O.to_bits(q8), want_bits)
 
 
+@pytest.mark.parametrize("computed,chunks", [
+    ([0, 0], [16, 48]),          # runs and token blocks start together
+    ([5, 13, 30], [16, 35, 45]), # runs cross the 16-token blocks
+    ([9, 0, 7], [7, 32, 25]),    # a sequence ends with a block, positions meet the next one's
+    ([15] * 20, [5] * 20),       # four or more runs a block
+])
+def test_amax_append_run_boundaries(gpu, computed, chunks):
+    # the token before a 16-token block decides whether a run continues into it
+    hkv, d = 2, 128
+    rng = np.random.default_rng(len(chunks))
+    tables, num_pages = random_tables(rng, [c + n for c, n in zip(computed, chunks)])
+    meta = prefill_metadata(tables, computed, chunks)
+    g = torch.Generator(device=gpu)
+    g.manual_seed(len(chunks))
+    q8 = torch.full((num_pages, 2, hkv, 16, d), 0x31, dtype=torch.uint8,
+                    device=gpu).view(torch.float8_e4m3fn)
+    scales = torch.full((num_pages, 2, hkv), 2.0 ** -9, device=gpu)
+    k, v = (_rows(g, meta.nnz, hkv, d, torch.bfloat16, gpu) for _ in range(2))
+    want_bits, want_sc, skipped = O.append_pages_e4m3_running(
+        O.to_bits(q8), scales.cpu(), k.cpu(), v.cpu(), meta.batch_indices, meta.positions,
+        meta.kv_indices, meta.kv_indptr)
+    _amax_append(gpu, meta, q8, scales, k, v)
+    assert skipped == 0
+    assert torch.equal(scales.cpu(), want_sc)
+    assert np.array_equal(O.to_bits(q8), want_bits)
+
+
 def test_amax_append_continues_partial_pages_and_zero_rows(gpu):
     rng = np.random.default_rng(3)
     hkv, d = 8, 128
