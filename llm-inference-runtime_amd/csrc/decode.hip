@@ -27,8 +27,9 @@
 // one is computed (two register buffers of 16 KiB each, ping-pong).  Page
 // ids are scalar loads issued one buffer ahead of their use.
 //
-// K rows are read as 16-byte (bf16/fp16) or 8-byte (e4m3) pieces in the
-// MFMA A-operand layout (lane -> token row, 8 consecutive d).  V rows are
+// K rows are read as 16-byte pieces (e4m3 at D = 64: 8-byte ones) in the
+// MFMA A-operand layout (lane -> token row, 8 consecutive d per k-step; an e4m3
+// piece at D = 128 holds two k-steps' d, and Q is laid out to match).  V rows are
 // read as W = D/16 consecutive d per lane (lane n owns d in [W n, W n + W)),
 // which gives W PV tiles whose row m is d = W m + e; the 8 tokens a lane
 // needs for one tile come from its own 8 loads, repacked with bit ops.
@@ -178,7 +179,11 @@ struct DecodeTraits {
   static constexpr int ESZ = FP8 ? 1 : 2;
   static constexpr int KS = D / 32;          // QK k-steps per page
   static constexpr int W = D / 16;           // V elements per lane per token
-  static constexpr int KB = 8 * ESZ;         // K bytes per lane per k-step
+  // e4m3 at D = 128: one 16-byte K load per lane serves two k-steps (d order
+  // within the pair of steps permuted alike in Q, q_dim)
+  static constexpr bool KWIDE = FP8 && D == 128;
+  static constexpr int KL = KWIDE ? KS / 2 : KS;       // K loads per lane and page
+  static constexpr int KB = 8 * ESZ * (KWIDE ? 2 : 1);  // bytes of one
   static constexpr int VB = W * ESZ;         // V bytes per lane per token
   static constexpr int PAGE_BYTES = kPage * D * ESZ;
   // page pairs per register buffer: 16 KiB of K/V per buffer, except e4m3
@@ -187,21 +192,27 @@ struct DecodeTraits {
   // the 70B-shaped e4m3 batch in 279 us against 282 us with two
   static constexpr int NP =
       (FP8 && D == 128) ? 1 : ((kPage * D * ESZ * 2 * 2 >= 16384) ? 1 : 2);
+  // first of the 8 d of Q and K in lane group G at k-step ks
+  static __device__ __forceinline__ int q_dim(int ks, int G) {
+    return KWIDE ? 64 * (ks >> 1) + 16 * G + 8 * (ks & 1) : 32 * ks + 8 * G;
+  }
   using KRaw = typename RawT<KB>::type;
   using VRaw = typename RawT<VB>::type;
-  // Cache policy of the K/V loads.  16-bit pools stream (non-temporal); e4m3
-  // pools load with the default policy.  Measured on the decode steps, with
-  // pools rotated past the Infinity Cache: the 70B-shaped e4m3 batch takes
-  // 225 us with the default policy against 276 us streamed, while the bf16
-  // long-context and TinyLlama steps take 1946 / 66 us with it against
-  // 1799 / 58 us streamed.
-  static constexpr int KV_POLICY = FP8 ? kCachePolicyDefault : kCachePolicyStream;
+  // Cache policy of the K/V loads: streamed (non-temporal) where every wave
+  // instruction covers at least 64 consecutive bytes of a row, default where
+  // its K loads cover 32 (e4m3 at D = 64): streamed, such a line is fetched
+  // for each of its parts.  Measured with pools rotated past the Infinity
+  // Cache: the bf16 long-context and TinyLlama steps take 1799 / 58 us
+  // streamed against 1946 / 66 us; the 70B-shaped e4m3 batch (1.26 GB) with
+  // 8-byte K loads 276 us streamed and 211 us default, with the 16-byte ones
+  // streamed 196 us (6.4 TB/s).
+  static constexpr int KV_POLICY = FP8 && D == 64 ? kCachePolicyDefault : kCachePolicyStream;
 };
 
 template <int D, bool BF16, bool FP8>
 struct Stage {
   using Tr = DecodeTraits<D, BF16, FP8>;
-  typename Tr::KRaw k[2][Tr::KS];
+  typename Tr::KRaw k[2][Tr::KL];
   typename Tr::VRaw v[8];
   int ntok[2];
   float kscale[2], vscale[2];
@@ -300,9 +311,9 @@ __device__ __forceinline__ void load_pair(Stage<D, BF16, FP8>& st,
     const __amdgpu_buffer_rsrc_t rk = make_rsrc(kbase, bytes);
     const __amdgpu_buffer_rsrc_t rv = make_rsrc(vbase, bytes);
 #pragma unroll
-    for (int ks = 0; ks < Tr::KS; ++ks)
+    for (int ks = 0; ks < Tr::KL; ++ks)
       st.k[pi][ks] = RawT<Tr::KB>::template load<Tr::KV_POLICY>(
-          rk, (uint32_t)((n * D + 32 * ks + 8 * G) * Tr::ESZ));
+          rk, (uint32_t)(n * D * Tr::ESZ + (4 * ks + G) * Tr::KB));
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       st.v[pi * 4 + r] = RawT<Tr::VB>::template load<Tr::KV_POLICY>(
@@ -343,10 +354,11 @@ __device__ __forceinline__ void compute_pairs(const Stage<D, BF16, FP8> (&st)[NP
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < Tr::KS; ++ks) {
-        const typename Tr::KRaw kr = st[k].k[pi][ks];
+        const typename Tr::KRaw kr = st[k].k[pi][Tr::KWIDE ? ks >> 1 : ks];
         u32x4 a;
         if constexpr (FP8) {
-          a = e4m3x8_to_16<BF16>(kr[0], kr[1]);
+          const int at = Tr::KWIDE ? 2 * (ks & 1) : 0;
+          a = e4m3x8_to_16<BF16>(kr[at], kr[at + 1]);
         } else {
           a = kr;
         }
@@ -592,7 +604,7 @@ __global__ void __launch_bounds__(256, 1) decode_kernel(DecodeParams p) {
 #pragma unroll
       for (int ks = 0; ks < D / 32; ++ks) {
         u32x4 z = {0u, 0u, 0u, 0u};
-        if (hv) z = *reinterpret_cast<const u32x4*>(qrow + 32 * ks + 8 * G);
+        if (hv) z = *reinterpret_cast<const u32x4*>(qrow + Tr::q_dim(ks, G));
         qf[ks] = z;
       }
     }
@@ -606,7 +618,7 @@ __global__ void __launch_bounds__(256, 1) decode_kernel(DecodeParams p) {
 #pragma unroll
       for (int ks = 0; ks < D / 64; ++ks) {
         float cs[8], sn[8];
-        rope_table8<D>(rope_tab, 32 * ks + 8 * G, cs, sn);
+        rope_table8<D>(rope_tab, Tr::q_dim(ks, G), cs, sn);
         rope8<BF16>(qf[ks], qf[ks + D / 64], cs, sn);
       }
     }
@@ -1074,7 +1086,7 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
         p.q + (int64_t)(b < 0 ? 0 : b) * p.q_sn + (int64_t)(h * g + (hv ? n : 0)) * p.q_sh;
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks)
-      qtmp[k][ks] = *reinterpret_cast<const u32x4*>(qrow + 32 * ks + 8 * G);
+      qtmp[k][ks] = *reinterpret_cast<const u32x4*>(qrow + Tr::q_dim(ks, G));
   }
 
   // with p.deterministic (the default) wave w takes chunks w, w + 4, w + 8,
@@ -1126,7 +1138,7 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
 #pragma unroll
           for (int ks = 0; ks < D / 64; ++ks) {
             float cs[8], sn[8];
-            rope_table8<D>(L.rope[wave], 32 * ks + 8 * G, cs, sn);
+            rope_table8<D>(L.rope[wave], Tr::q_dim(ks, G), cs, sn);
             rope8<BF16>(qtmp[k][ks], qtmp[k][ks + D / 64], cs, sn);
           }
         }
