@@ -89,25 +89,28 @@ constexpr int kPrefillDevMaxBatch = 4096;
 constexpr int kPrefillDevSortMax = 1024;
 // Split-KV prefill: a step whose q-tiles x KV heads are fewer than the CUs
 // cuts the KV tiles of its long q-tiles into pieces, one workgroup each, merged
-// by a second launch.  The longest tile of t_max KV tiles gets P pieces of
-// ceil(t_max / P), every other tile pieces of at most that many: P is the
-// largest (up to kPrefillSplitMaxPieces) whose pieces all run at once, with
-// at least kPrefillSplitMinTiles KV tiles a piece.
+// by a second launch.  The longest tile of t_max KV tiles gets P pieces (up to
+// kPrefillSplitMaxPieces) of at most L = ceil(t_max / P) >=
+// kPrefillSplitMinTiles, every other tile pieces of at most L, and all pieces
+// run at once (at most `slots` of them per KV head, one workgroup per CU).  P
+// is the one with the least estimated time, if that beats the whole tiles'.
+//
+// The estimate (half microseconds x slots, D = 128; at D = 64 all of it is
+// about a third less): a KV tile takes 1.5 us on a mostly idle GPU and 2 us on a
+// full one, and the partials and the merge launch 5 us plus 6 us on a full GPU.
+// Measured on steps of 32/8 heads at D = 128, whole and cut: 1 x 8 workgroups
+// of 16 KV tiles 30.7 and 12.5 us; 8 x 8 of 13 28.7 and 24.8 us, of 133 200
+// and 85 us; 16 x 8 of 17 38.5 and 41.7 us (kept whole), of 24 45.7 and 44.7 us,
+// of 141 212 and 157 us.
 constexpr int kPrefillSplitMaxPieces = 128;
-constexpr int kPrefillSplitMinTiles = 4;
+constexpr int kPrefillSplitMinTiles = 3;
 constexpr int kPrefillKvTile = 64;
-// Whether pieces of at most `len` KV tiles, `pieces` of them on `slots` places
-// per KV head, beat the longest workgroup's t_max: a KV tile takes 1.5 us on a
-// mostly idle GPU and 2 us on a full one, and the partials and the merge
-// launch 5 us plus 6 us on a full GPU (D = 128; at D = 64 all of it is about
-// a third less).  Measured on steps of 32/8 heads, D = 128, one tile per
-// sequence unless stated: 1 x 8 workgroups of 16 KV tiles 30.7 us whole, 12.5
-// us cut; 8 x 8 of 13 28.7 and 24.8 us, of 133 200 and 85 us; 16 x 8 of 17
-// 38.5 and 41.7 us (kept whole), of 24 45.7 and 44.7 us, of 141 212 and 157 us.
-inline __host__ __device__ bool prefill_split_pays(int t_max, int len, int64_t pieces,
+inline __host__ __device__ int64_t prefill_split_cost(int len, int64_t pieces, int64_t slots) {
+  return (3 * slots + pieces) * len + 10 * slots + 12 * pieces;
+}
+inline __host__ __device__ bool prefill_split_pays(int t_max, int len, int64_t cost,
                                                    int64_t slots) {
-  return t_max - len >= 6 &&
-         3 * slots * t_max > (3 * slots + pieces) * len + 10 * slots + 12 * pieces;
+  return t_max - len >= 4 && cost < 3 * slots * t_max;
 }
 
 // Workspace of a split prefill plan, from the workspace start: the cut tiles'

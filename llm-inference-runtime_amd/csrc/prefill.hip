@@ -862,7 +862,7 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
   static_assert(kPrefillPlanThreads == 8 * kPrefillSplitMaxPieces, "8 threads per cut");
   __shared__ int kv_tiles[kPrefillDevSortMax];  // KV tiles, then first entry, by list place
   __shared__ int t_max_s;
-  __shared__ unsigned best_s;  // the best cut's P << 16 | pieces
+  __shared__ unsigned long long best_s;  // the best cut's cost << 8 | P
   const int t = threadIdx.x;
   const int B = min(max(a.batch_size, 0), kPrefillDevMaxBatch);
   auto qo_len = [&](int b) {
@@ -938,7 +938,7 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
     }
     if (t == 0) {
       t_max_s = 0;
-      best_s = 0;
+      best_s = ~0ull;
     }
     __syncthreads();
     if (t < n_tiles) {
@@ -962,12 +962,14 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
 #pragma unroll
       for (int off = 1; off < 8; off <<= 1) count += __shfl_xor(count, off);
       if (P > 1 && lp >= kPrefillSplitMinTiles && count <= a.slots && (t & 7) == 0)
-        atomicMax(&best_s, (unsigned)P << 16 | (unsigned)count);
+        atomicMin(&best_s,
+                  (unsigned long long)prefill_split_cost(lp, count, a.slots) << 8 | (unsigned)P);
       __syncthreads();
-      const int best = (int)(best_s >> 16);
-      if (best > 1) {
-        const int lb = (t_max + best - 1) / best;
-        if (prefill_split_pays(t_max, lb, (int)(best_s & 0xffff), a.slots)) len = lb;
+      const unsigned long long best = best_s;
+      if (best != ~0ull) {
+        const int P = (int)(best & 0xff);
+        const int lb = (t_max + P - 1) / P;
+        if (prefill_split_pays(t_max, lb, (int64_t)(best >> 8), a.slots)) len = lb;
       }
     }
     if (len > 0) {

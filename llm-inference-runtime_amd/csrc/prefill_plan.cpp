@@ -44,20 +44,21 @@ static int64_t prefill_split_slots(int hkv) {
 static int prefill_piece_tiles(const std::vector<int>& tiles, int64_t slots) {
   if (tiles.empty() || (int64_t)tiles.size() > slots) return 0;
   const int t_max = *std::max_element(tiles.begin(), tiles.end());
-  auto len = [&](int p) { return (t_max + p - 1) / p; };
-  auto count = [&](int p) {
+  int best = 0;
+  int64_t best_cost = 0;
+  for (int p = 2; p <= kPrefillSplitMaxPieces; ++p) {
+    const int len = (t_max + p - 1) / p;
+    if (len < kPrefillSplitMinTiles) break;
     int64_t n = 0;
-    for (int t : tiles) n += t > 0 ? (t + len(p) - 1) / len(p) : 1;
-    return n;
-  };
-  auto fits = [&](int p) { return len(p) >= kPrefillSplitMinTiles && count(p) <= slots; };
-  int lo = 1, hi = kPrefillSplitMaxPieces;  // more pieces only ever take more slots
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) / 2;
-    if (t_max > 0 && fits(mid)) lo = mid;
-    else hi = mid - 1;
+    for (int t : tiles) n += t > 0 ? (t + len - 1) / len : 1;
+    if (n > slots) break;  // more pieces only ever take more slots
+    const int64_t cost = prefill_split_cost(len, n, slots);
+    if (best == 0 || cost < best_cost) {
+      best = len;
+      best_cost = cost;
+    }
   }
-  return lo > 1 && prefill_split_pays(t_max, len(lo), count(lo), slots) ? len(lo) : 0;
+  return best > 0 && prefill_split_pays(t_max, best, best_cost, slots) ? best : 0;
 }
 
 // The device side of a split plan: work list, merge list and partials.
