@@ -686,7 +686,7 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
 // (Hkv = 8).
 struct PrefillMergeArgs {
   const PrefillMerge* merges;
-  const int32_t* n_merge;
+  const int32_t* n_merge;  // null: `cap` of them
   int32_t cap, batch_size, hq, hkv, g, n_slots;
   const int32_t* qo_indptr;
   const float* po;
@@ -708,7 +708,7 @@ __global__ void __launch_bounds__(kWave * kPrefillMergeWaves)
   const int lane = threadIdx.x & 63;
   const int wave = uniform(threadIdx.x >> 6);
   const int col = lane & 31, half = lane >> 5;
-  const int n_merge = min(uniform(load_invariant(a.n_merge)), a.cap);
+  const int n_merge = a.n_merge ? min(uniform(load_invariant(a.n_merge)), a.cap) : a.cap;
   const int64_t units = (int64_t)n_merge * BLKS * DT * a.hkv;
   for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
     const int h = (int)(u % a.hkv);
@@ -723,10 +723,11 @@ __global__ void __launch_bounds__(kWave * kPrefillMergeWaves)
     // (uniform over the workgroup, as every condition up to the barriers)
     if (b < 0 || b >= a.batch_size || q_lo < 0 || slot0 < 0 || n < 1 || n > a.n_slots - slot0)
       continue;
+    const int q_end = uniform(load_invariant(mp + 2));
+    if (32 * blk >= (q_end - q_lo) * a.g) continue;
+    // used after the partials' loads are issued
     const int qo_start = uniform(load_invariant(a.qo_indptr + b));
-    const int q_hi = min(uniform(load_invariant(mp + 2)),
-                         uniform(load_invariant(a.qo_indptr + b + 1)) - qo_start);
-    if (32 * blk >= (q_hi - q_lo) * a.g) continue;
+    const int q_hi = min(q_end, uniform(load_invariant(a.qo_indptr + b + 1)) - qo_start);
     float M = -INFINITY, den = 0.f;
     f32x4 num[4];
 #pragma unroll
@@ -1156,7 +1157,8 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   // host plans know their cut tiles; a device plan's are at most half its
   // slots, and its merge workgroups find out how many there are
   const int cap = plan->implicit ? plan->n_slots / 2 : plan->n_merge;
-  PrefillMergeArgs m{static_cast<const PrefillMerge*>(plan->merge_dev), split_count(plan), cap,
+  PrefillMergeArgs m{static_cast<const PrefillMerge*>(plan->merge_dev),
+                     plan->implicit ? split_count(plan) : nullptr, cap,
                      plan->batch_size, plan->hq, plan->hkv, p.g, plan->n_slots, qo_indptr,
                      plan->partial_o, plan->partial_lse, p.out, lse};
   const int64_t units = (int64_t)cap * (kPrefillRows / 32) * (plan->d / 32) * plan->hkv;
