@@ -42,7 +42,7 @@
 namespace pa {
 
 struct PrefillParams {
-  const void* items;  // PrefillItem, or PrefillPiece (SPLIT)
+  const PrefillItem* items;  // SPLIT: PrefillPiece entries
   int32_t n_items, batch_size;
   const uint16_t* q;
   int64_t q_sn, q_sh;
@@ -313,8 +313,9 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
   // a work list that does not match this launch is skipped, never followed
   // (every condition is uniform over the workgroup)
   if (item >= p.n_items) return;
-  constexpr int ITEM_INTS = (SPLIT ? sizeof(PrefillPiece) : sizeof(PrefillItem)) / 4;
-  const int32_t* itp = static_cast<const int32_t*>(p.items) + (int64_t)item * ITEM_INTS;
+  const int32_t* itp = reinterpret_cast<const int32_t*>(p.items + item);
+  if constexpr (SPLIT)
+    itp = reinterpret_cast<const int32_t*>(reinterpret_cast<const PrefillPiece*>(p.items) + item);
   const int b = uniform(load_invariant(itp + 0));
   if (b < 0 || b >= p.batch_size) return;
   const int qo_start = uniform(load_invariant(p.qo_indptr + b));
@@ -1118,7 +1119,7 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   if (num_pages < 0 || num_indices < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: negative sizes", who);
   PrefillParams p;
-  p.items = plan->items_dev;
+  p.items = static_cast<const PrefillItem*>(plan->items_dev);
   p.n_items = plan->n_items;
   p.batch_size = plan->batch_size;
   p.q = static_cast<const uint16_t*>(q);
