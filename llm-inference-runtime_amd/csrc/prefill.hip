@@ -657,8 +657,9 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
               for (int i = 0; i < 4; ++i) w[i] = o[rb][dt][4 * i4 + i] * inv;
               *reinterpret_cast<f32x4*>(po + (4 * dt + i4) * 256) = w;
             }
+          // NaN where a score was NaN, for the merge to pass on
           if (half == 0)
-            p.partial_lse[blk * 32 + col] = l_tot > 0.f ? m[rb] + log2f(l_tot) : -INFINITY;
+            p.partial_lse[blk * 32 + col] = l_tot == 0.f ? -INFINITY : m[rb] + log2f(l_tot);
           continue;
         }
       }
@@ -702,7 +703,9 @@ __global__ void __launch_bounds__(64 * kPrefillWaves, 1) prefill_kernel(PrefillP
 }
 
 // Merge of the cut tiles of a split plan:
-// o = sum_k 2^(lse_k - M) o_k / sum_k 2^(lse_k - M) over a row's pieces.
+// o = sum_k 2^(lse_k - M) o_k / sum_k 2^(lse_k - M) over a row's pieces.  A
+// piece with a NaN lse makes the row NaN with lse = -inf, as the whole tile
+// writes it; a row that sees nothing has den = 0 and num = 0.
 // Unit: 32 rows x 32 d of one cut tile and KV head; a workgroup's four waves
 // take pieces w, w + 4, ... (kPieces loads of each lane at a time), and add
 // up through LDS in wave order.  Bound by the partials' bytes (P x 2 x 128 KiB
@@ -806,18 +809,16 @@ __global__ void __launch_bounds__(kWave * kPrefillMergeWaves)
     for (int w = 0; w < NW; ++w) M = fmaxf(M, s_m[w][lane]);
     den = 0.f;
     f32x4 o4 = {0.f, 0.f, 0.f, 0.f};
-    if (M != -INFINITY) {
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const float mw = s_m[w][lane];
-        const float wt = mw == -INFINITY ? 0.f : exp2f(mw - M);
-        den = fmaf(wt, s_den[w][lane], den);
-        const f32x4 x = s_num[w][wave][lane];
+    for (int w = 0; w < NW; ++w) {
+      const float mw = s_m[w][lane];
+      const float wt = mw == -INFINITY ? 0.f : exp2f(mw - M);
+      den = fmaf(wt, s_den[w][lane], den);
+      const f32x4 x = s_num[w][wave][lane];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o4[e] = fmaf(wt, x[e], o4[e]);
-      }
-      o4 *= 1.f / den;
+      for (int e = 0; e < 4; ++e) o4[e] = fmaf(wt, x[e], o4[e]);
     }
+    if (den != 0.f) o4 *= 1.f / den;
     const int row = 32 * blk + col;
     const int qi = q_lo + row / a.g;
     if (qi < q_hi) {
@@ -827,7 +828,7 @@ __global__ void __launch_bounds__(kWave * kPrefillMergeWaves)
       w2[1] = pack2_16<BF16>(o4[2], o4[3]);
       *reinterpret_cast<u32x2*>(a.out + orow * D + 32 * dt + 8 * wave + 4 * half) = w2;
       if (a.lse && dt == 0 && wave == 0 && half == 0)
-        a.lse[orow] = M != -INFINITY ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
+        a.lse[orow] = den > 0.f ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
     }
     __syncthreads();  // the sums are read before the next unit writes its own
   }

@@ -212,3 +212,35 @@ def test_prefill_split_kv(gpu, monkeypatch, step, d, hq, hkv, fp8, causal):
     assert not torch.equal(lse, lse_w)  # the large workspace's plan was cut
     assert max_err(out_w, ref_o) <= tol
     assert lse_err(lse_w, ref_l) <= TOL_LSE
+
+
+@pytest.mark.parametrize("d,hq,hkv,fp8", [(128, 32, 8, False), (64, 32, 4, False),
+                                          (64, 32, 4, True)])
+@pytest.mark.parametrize("where", ["q_nan", "q_inf", "k_nan", "v_nan"])
+def test_prefill_split_kv_not_finite(gpu, monkeypatch, d, hq, hkv, fp8, where):
+    # a value that is not finite reaches the same outputs and lse whether the
+    # KV range is cut or not: in every piece (a q row) or in one (a K or V row)
+    if fp8 and where != "q_nan":
+        pytest.skip("the pool's rows are finite codes")
+    monkeypatch.delenv("PAGEDATTN_PREFILL_SPLIT", raising=False)
+    meta, pool, q = prefill_case(gpu, [3000, 2000], [70, 20], hq, hkv, d, seed=d)
+    page = int(meta.kv_indices[40])
+    if where[0] == "q":
+        q[33, 1, 0] = float(where[2:])
+    else:
+        pool[page, "kv".index(where[0]), :, 3] = float("nan")
+    scales = None
+    if fp8:
+        pool, scales = pagedattn.quantize_pages_e4m3(pool)
+    out, lse = run_prefill(gpu, meta, pool, q, hq, hkv, d, kv_scales=scales)
+    small = torch.zeros(1 << 16, dtype=torch.uint8, device=gpu)
+    out_w, lse_w = run_prefill(gpu, meta, pool, q, hq, hkv, d, kv_scales=scales, ws=small)
+    bad = torch.isnan(out_w)
+    assert bad.any() and not bad.all()
+    assert torch.equal(torch.isnan(out), bad)
+    assert max_err(torch.where(bad, 0, out), torch.where(bad, 0, out_w).float().cpu()) <= TOL_BF16
+    none = torch.isinf(lse_w)
+    assert torch.equal(torch.isinf(lse), none) and not torch.isnan(lse).any()
+    assert none.any() == (where != "v_nan")
+    assert not torch.equal(lse[~none], lse_w[~none])  # the large workspace's plan was cut
+    assert float((lse - lse_w)[~none].abs().max()) <= TOL_LSE
