@@ -557,7 +557,10 @@ __device__ __forceinline__ void write_item_output(const DecodeParams& p, int b, 
       for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int e = 0; e < W; ++e) prow[W * (4 * G + r) + e] = sm.o[e][r] * inv;
-      if (G == 0) p.partial_lse[(int64_t)slot * g + n] = lse2;
+      // NaN where a score was NaN, for the merge to pass on
+      if (G == 0)
+        p.partial_lse[(int64_t)slot * g + n] =
+            l_tot == 0.f ? -INFINITY : sm.m + log2f(l_tot);
     }
   }
 }
@@ -1318,7 +1321,9 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
 // 2^(lse - M) o, out = num / den.  Pieces s, s + 8, s + 16, ... form class
 // s mod 8; a wave sums a class, kMergeBatch loads at a time, and the classes
 // are added in order, so the bits depend on the piece count alone and not on
-// the workgroup's waves (any number from D / 64 to 8).
+// the workgroup's waves (any number from D / 64 to 8).  A piece with a NaN lse
+// makes the row NaN with lse = -inf, as an uncut item writes it; with no score
+// at all den and num are 0.
 //
 // Bound by the latency of dependent loads, not by bytes (a partial row is
 // 256-512 B): one thread per d walking the pieces four at a time took 24
@@ -1332,9 +1337,9 @@ constexpr int kMergeBatch = 8;
 template <bool BF16>
 __device__ __forceinline__ void merge_write(float M, float num, float den, int dd, uint16_t* orow,
                                             float* lse) {
-  orow[dd] = f2h<BF16>(M != -INFINITY ? num / den : 0.f);
+  orow[dd] = f2h<BF16>(den != 0.f ? num / den : num);
   if (lse && dd == 0)
-    *lse = M != -INFINITY ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
+    *lse = den > 0.f ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
 }
 
 template <bool BF16, int D, typename SlotOf>
@@ -1358,13 +1363,11 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
       }
       M = fmaxf(M, lv[s]);
     }
-    if (M != -INFINITY) {
 #pragma unroll
-      for (int s = 0; s < kMergeClasses; ++s) {
-        const float wt = lv[s] == -INFINITY ? 0.f : exp2f(lv[s] - M);
-        den += wt;
-        num = fmaf(wt, ov[s], num);
-      }
+    for (int s = 0; s < kMergeClasses; ++s) {
+      const float wt = lv[s] == -INFINITY ? 0.f : exp2f(lv[s] - M);
+      den += wt;
+      num = fmaf(wt, ov[s], num);
     }
     merge_write<BF16>(M, num, den, dd, orow, lse);
     return;
@@ -1394,7 +1397,6 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
       float Mb = M;
 #pragma unroll
       for (int k = 0; k < kMergeBatch; ++k) Mb = fmaxf(Mb, lv[k]);
-      if (Mb == -INFINITY) continue;
       const float r = M == -INFINITY ? 0.f : exp2f(M - Mb);
       den *= r;
 #pragma unroll
@@ -1420,13 +1422,11 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
   float M = -INFINITY, den = 0.f, num = 0.f;
 #pragma unroll
   for (int w = 0; w < kMergeClasses; ++w) M = fmaxf(M, s_m[w]);
-  if (M != -INFINITY) {
 #pragma unroll
-    for (int w = 0; w < kMergeClasses; ++w) {
-      const float wt = s_m[w] == -INFINITY ? 0.f : exp2f(s_m[w] - M);
-      den = fmaf(wt, s_den[w], den);
-      num = fmaf(wt, s_num[w][dd], num);
-    }
+  for (int w = 0; w < kMergeClasses; ++w) {
+    const float wt = s_m[w] == -INFINITY ? 0.f : exp2f(s_m[w] - M);
+    den = fmaf(wt, s_den[w], den);
+    num = fmaf(wt, s_num[w][dd], num);
   }
   merge_write<BF16>(M, num, den, dd, orow, lse);
 }

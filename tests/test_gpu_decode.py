@@ -489,3 +489,34 @@ def test_decode_fused_append_counts(gpu):
         torch.cuda.synchronize()
         assert np.array_equal(O.to_bits(pb), want), split
         assert ws[:8].view(torch.int32).tolist() == [skipped, clamped], split
+
+
+@pytest.mark.parametrize("d,fp8", [(64, False), (128, False), (128, True)])
+@pytest.mark.parametrize("split_pages", [8, 64])
+@pytest.mark.parametrize("where", ["q_nan", "k_nan", "v_nan"])
+def test_decode_merge_not_finite(gpu, d, fp8, split_pages, where):
+    # a value that is not finite reaches the same outputs and lse whether the
+    # sequence is cut or not, up to 8 pieces a row (64-page chunks) and past
+    # it: in every piece (a q row) or in one (a K or V row)
+    if fp8 and where != "q_nan":
+        pytest.skip("the pool's rows are finite codes")
+    hq, hkv = 8, 2
+    meta, pool, q = decode_case(gpu, [3000, 700, 3000], hq, hkv, d, seed=d)
+    if where == "q_nan":
+        q[0, 5] = float("nan")
+    else:
+        pool[int(meta.kv_indices[40]), "kv".index(where[0]), :, 3] = float("nan")
+    scales = None
+    if fp8:
+        pool, scales = pagedattn.quantize_pages_e4m3(pool)
+    out_w, lse_w = run_decode(gpu, meta, pool, q, hq, hkv, d, split_pages=-1, kv_scales=scales)
+    out, lse = run_decode(gpu, meta, pool, q, hq, hkv, d, split_pages=split_pages,
+                          kv_scales=scales)
+    bad = torch.isnan(out_w)
+    assert bad.any() and not bad.all()
+    assert torch.equal(torch.isnan(out), bad)
+    assert max_err(torch.where(bad, 0, out), torch.where(bad, 0, out_w).float().cpu()) <= TOL_BF16
+    none = torch.isinf(lse_w)
+    assert torch.equal(torch.isinf(lse), none) and not torch.isnan(lse).any()
+    assert none.any() == (where != "v_nan")
+    assert float((lse - lse_w)[~none].abs().max()) <= TOL_LSE
