@@ -273,7 +273,7 @@ int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,
   const int64_t slots = prefill_split_slots(num_kv_heads);
   const int64_t entries = std::max(cap, slots);
   const PrefillSplitLayout lay = prefill_split_layout(entries, slots, num_kv_heads, head_dim);
-  if (prefill_splitting() && slots >= 2 && slots <= kPrefillDevSortMax &&
+  if (cap > 0 && prefill_splitting() && slots >= 2 && slots <= kPrefillDevSortMax &&
       lay.end <= workspace_bytes && entries * num_kv_heads <= INT32_MAX) {
     plan->n_items = (int)entries;
     plan->q_cap = (int)cap;

@@ -86,6 +86,24 @@ def test_abi_rejects_bad_arguments_without_device():
     assert rc == 1
 
 
+@pytest.mark.parametrize("ws_bytes", [1 << 16, 1 << 27])
+def test_empty_device_prefill_plan_runs(ws_bytes):
+    # no sequences and no tokens: nothing to launch, whatever the workspace
+    # (never touched here) could hold
+    lib = _lib.lib()
+    plan = lib.pagedattn_plan_create()
+    ws = ctypes.c_void_p(1 << 20)
+    args = (None, 0, 0, _lib.BF16, None, None, _lib.BF16, None, 0, None, 0, None, None, None,
+            None, 1, ctypes.c_float(1.0), None)
+    try:
+        for tokens, rc in ((0, 0), (1, 1)):  # with a tile to run, null pointers are an error
+            assert lib.pagedattn_prefill_plan_device(plan, 0, 32, 8, 128, 16, tokens, ws,
+                                                     ws_bytes) == 0
+            assert lib.pagedattn_prefill_run(plan, *args) == rc, lib.pagedattn_last_error()
+    finally:
+        lib.pagedattn_plan_destroy(plan)
+
+
 def test_wrappers_require_device_tensors():
     ws = torch.zeros(1024, dtype=torch.uint8)
     with pytest.raises(ValueError, match="device"):
