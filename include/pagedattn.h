@@ -248,11 +248,27 @@ int pagedattn_build_paged_metadata(const int32_t* block_tables, int64_t table_st
  * prefill runs dropped because they exceeded the plan's capacity (their
  * output rows are left unwritten).
  *
- * Runs whose plan cuts KV ranges write their split partials into the
- * workspace, so two runs of one plan must not overlap on the GPU (runs of
- * one stream never do); give concurrent streams a plan and a workspace each. */
+ * Overlapping runs.  Shared-item decode plans and prefill plans are only read
+ * by their runs, so runs of one plan may overlap on the GPU (several streams);
+ * a device prefill plan's runs write its lists, the same values each time while
+ * its metadata stays the same.
+ * Split decode plans and device decode plans of the split kind keep their
+ * partials in the workspace: give concurrent streams a plan and a workspace
+ * each.  Plans with pagedattn_plan_scratch_bytes > 0 (below) may overlap too. */
 pagedattn_plan* pagedattn_plan_create(void);
 void pagedattn_plan_destroy(pagedattn_plan* plan);
+
+/* Scratch of the pagedattn_*_run_scratch calls, which have no counterpart in
+ * the reference.  Work that leaves CUs idle when kept whole (prefill steps of
+ * few q-tiles, decode batches of fewer (sequence, KV head) items than CUs) is
+ * planned twice: whole, and with the KV ranges cut into pieces that a second
+ * launch merges.  The pieces' partials belong to one run, so the run brings the
+ * memory: device scratch of at least this many bytes (256-byte aligned, any
+ * contents, used in stream order until the run has ended; at most the
+ * workspace's size, which bounds it at plan time).  Runs without scratch, and
+ * the calls without the argument, take the whole form.  0: the plan has one
+ * form, and scratch is ignored.  The two forms round differently. */
+size_t pagedattn_plan_scratch_bytes(const pagedattn_plan* plan);
 
 int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
                           const int32_t* kv_last_page_len_host,
@@ -317,9 +333,11 @@ int pagedattn_decode_plan_device_update(pagedattn_plan* plan, const int32_t* kv_
  * split_pages = 0 takes a shared plan when its busiest CU carries at most
  * PAGEDATTN_DECODE_SHARED_SLACK_KB (environment, default 96, or 120 for fewer
  * items than CUs) KiB plus PAGEDATTN_DECODE_SHARED_SLACK_PCT (default 4)
- * percent of the mean more K/V than the mean over all CUs (a workspace too
- * small for the split's partials keeps a plan that is balanced over the CUs
- * it uses); PAGEDATTN_DECODE_SHARED=0 / =1 turns that off / takes one
+ * percent of the mean more K/V than the mean over all CUs.  A plan that is
+ * balanced over fewer CUs is a split one for runs with scratch
+ * (pagedattn_plan_scratch_bytes) and a shared one for runs without (and
+ * altogether where the workspace could not hold the split's partials);
+ * PAGEDATTN_DECODE_SHARED=0 / =1 turns that off / takes one
  * whenever it fits.  A shared plan's waves take fixed page pairs, so repeated
  * runs give identical bits; PAGEDATTN_DECODE_DETERMINISTIC=0 (read at plan
  * time) lets them claim pairs in arrival order instead, which balances the
@@ -393,16 +411,32 @@ int pagedattn_decode_run_rope_append(
     const int32_t* kv_last_page_len, void* out, float* lse, float sm_scale,
     void* stream);
 
+/* The three decode runs with scratch: pagedattn_decode_run where append_key and
+ * append_value are NULL, else pagedattn_decode_run_append, or with rope != 0
+ * pagedattn_decode_run_rope_append.  scratch NULL is the call without it. */
+int pagedattn_decode_run_scratch(
+    const pagedattn_plan* plan, const void* q, int64_t q_stride_n,
+    int64_t q_stride_h, int32_t q_dtype, const void* append_key,
+    const void* append_value, int64_t k_stride_n, int64_t k_stride_h,
+    int64_t v_stride_n, int64_t v_stride_h, int32_t rope,
+    const int32_t* positions, float rope_scale, float rope_theta,
+    void* paged_kv_cache, int32_t kv_dtype, const float* kv_scales,
+    int32_t num_pages, const int32_t* kv_indices, int32_t num_indices,
+    const int32_t* kv_indptr, const int32_t* kv_last_page_len, void* out,
+    float* lse, float sm_scale, void* scratch, size_t scratch_bytes,
+    void* stream);
+
 /* BatchPrefillWithPagedKVCacheWrapper.begin_forward(qo_indptr, kv_indptr,
  *     kv_indices, kv_last_page_len, Hq, Hkv, D, page_size, q_data_type)
  *     (src/models/llama.py:86-116).  Host copies of the indptr arrays.
  * q-tiles of at most half a workgroup's rows are planned as pairs of KV
  * heads sharing one workgroup when num_kv_heads is even (same output bits);
  * PAGEDATTN_PREFILL_PAIR=0, read at plan time, plans every tile alone.
- * Steps with fewer q-tiles x KV heads than CUs cut the KV range of their long
- * tiles into pieces merged by a second launch, where the workspace holds the
- * partials (about 34 MiB at 256 CUs and D = 128, half at D = 64);
- * PAGEDATTN_PREFILL_SPLIT=0, read at plan time, keeps every tile whole. */
+ * Steps with fewer q-tiles x KV heads than CUs may also get a list that cuts
+ * the KV range of their long tiles into pieces merged by a second launch
+ * (pagedattn_plan_scratch_bytes), where the workspace is at least as large as
+ * the partials of one piece per CU (32.3 MiB at 256 CUs and D = 128, half at
+ * D = 64); PAGEDATTN_PREFILL_SPLIT=0, read at plan time, keeps every tile whole. */
 int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
                            const int32_t* kv_indptr_host,
                            const int32_t* kv_last_page_len_host,
@@ -421,10 +455,10 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
  * exactly as pagedattn_prefill_plan does (same pairing and pieces, up to 1024
  * tiles ordered longest first), into the workspace, then the attention over
  * the plan's fixed capacity of ceil(max_qo_tokens / q_tile) + batch_size tiles
- * (at least one workgroup per CU where pieces may be cut, and then the merge
- * launch); entries past the run's tiles return at once.  The outputs equal
- * those of a host plan bit for bit (whose workspace, like this one, holds the
- * partials, or does not).  Tiles beyond the capacity (a run with more than
+ * (a run with scratch: at least one workgroup per CU, then the merge launch);
+ * entries past the run's tiles return at once.  The outputs equal those of a
+ * host plan with a workspace of the same size, run like this one with or
+ * without scratch, bit for bit.  Tiles beyond the capacity (a run with more than
  * max_qo_tokens query tokens) are skipped and counted at byte 12 of the
  * workspace.  batch_size <= 4096. */
 int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,
@@ -460,6 +494,19 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
                           const int32_t* kv_last_page_len, void* out,
                           float* lse, int32_t causal, float sm_scale,
                           void* stream);
+
+/* The same with scratch (pagedattn_plan_scratch_bytes); NULL is the call
+ * without it. */
+int pagedattn_prefill_run_scratch(const pagedattn_plan* plan, const void* q,
+                                  int64_t q_stride_n, int64_t q_stride_h,
+                                  int32_t q_dtype, const int32_t* qo_indptr,
+                                  const void* paged_kv_cache, int32_t kv_dtype,
+                                  const float* kv_scales, int32_t num_pages,
+                                  const int32_t* kv_indices, int32_t num_indices,
+                                  const int32_t* kv_indptr,
+                                  const int32_t* kv_last_page_len, void* out,
+                                  float* lse, int32_t causal, float sm_scale,
+                                  void* scratch, size_t scratch_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------
  * No counterpart in the reference (its pool dtype equals the model dtype,

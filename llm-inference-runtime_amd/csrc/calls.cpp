@@ -17,6 +17,7 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/util/Exception.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -27,10 +28,9 @@ namespace {
 // C entry points, bound by address so that this module shares the library
 // instance (and HIP runtime) the package has loaded.
 struct Entries {
-  decltype(&pagedattn_decode_run) decode_run;
-  decltype(&pagedattn_decode_run_append) decode_run_append;
-  decltype(&pagedattn_decode_run_rope_append) decode_run_rope_append;
-  decltype(&pagedattn_prefill_run) prefill_run;
+  decltype(&pagedattn_plan_scratch_bytes) scratch_bytes;
+  decltype(&pagedattn_decode_run_scratch) decode_run;
+  decltype(&pagedattn_prefill_run_scratch) prefill_run;
   decltype(&pagedattn_append_paged_kv_cache) append;
   decltype(&pagedattn_rope_append_paged_kv_cache) rope_append;
   decltype(&pagedattn_append_paged_kv_cache_e4m3_amax) append_amax;
@@ -184,6 +184,26 @@ struct Outputs {
   }
 };
 
+// The scratch of one run of a plan that cuts KV ranges: torch's caching
+// allocator hands it out per run and stream (and per captured graph), so runs of
+// one plan may overlap; freed when the call returns, it is reused in stream
+// order.  Without memory for it the run takes the plan's whole form.
+struct Scratch {
+  at::Tensor t;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  void get(const pagedattn_plan* plan, const at::Tensor& q) {
+    bytes = g_entry.scratch_bytes(plan);
+    if (!bytes) return;
+    try {
+      t = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte).requires_grad(false));
+      ptr = t.data_ptr();
+    } catch (const c10::OutOfMemoryError&) {
+      bytes = 0;
+    }
+  }
+};
+
 PyObject* general() { Py_RETURN_NOTIMPLEMENTED; }
 
 bool arg_count(Py_ssize_t n, Py_ssize_t want) {
@@ -246,23 +266,16 @@ PyObject* decode_run(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* op = o.out.data_ptr();
   float* lp = static_cast<float*>(o.lse_ptr);
   const int code = code16(*q);
+  const int64_t ks[2] = {append ? k->stride(0) : 0, append ? k->stride(1) : 0};
+  const int64_t vs[2] = {append ? v->stride(0) : 0, append ? v->stride(1) : 0};
+  Scratch scratch;
+  scratch.get(plan, *q);
   int rc;
   Py_BEGIN_ALLOW_THREADS
-  if (!append)
-    rc = g_entry.decode_run(plan, qp, q->stride(0), q->stride(1), code, pp, pool.code, scales,
-                            (int32_t)pool.pages, indices, (int32_t)n_ind, indptr, last, op, lp,
-                            (float)scale, stream);
-  else if (!rope)
-    rc = g_entry.decode_run_append(plan, qp, q->stride(0), q->stride(1), code, kp, vp,
-                                   k->stride(0), k->stride(1), v->stride(0), v->stride(1), pp,
-                                   pool.code, scales, (int32_t)pool.pages, indices,
-                                   (int32_t)n_ind, indptr, last, op, lp, (float)scale, stream);
-  else
-    rc = g_entry.decode_run_rope_append(
-        plan, qp, q->stride(0), q->stride(1), code, kp, vp, k->stride(0), k->stride(1),
-        v->stride(0), v->stride(1), pos, (float)rope_scale, (float)rope_theta, pp, pool.code,
-        scales, (int32_t)pool.pages, indices, (int32_t)n_ind, indptr, last, op, lp, (float)scale,
-        stream);
+  rc = g_entry.decode_run(plan, qp, q->stride(0), q->stride(1), code, kp, vp, ks[0], ks[1], vs[0],
+                          vs[1], rope, pos, (float)rope_scale, (float)rope_theta, pp, pool.code,
+                          scales, (int32_t)pool.pages, indices, (int32_t)n_ind, indptr, last, op,
+                          lp, (float)scale, scratch.ptr, scratch.bytes, stream);
   Py_END_ALLOW_THREADS
   return rc ? PyLong_FromLong(rc) : o.result();
   END_HANDLE_TH_ERRORS
@@ -299,11 +312,14 @@ PyObject* prefill_run(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const void* qp = q->data_ptr();
   void* pp = pool.ptr();
   void* op = o.out.data_ptr();
+  Scratch scratch;
+  scratch.get(plan, *q);
   int rc;
   Py_BEGIN_ALLOW_THREADS
   rc = g_entry.prefill_run(plan, qp, q->stride(0), q->stride(1), code16(*q), qo, pp, pool.code,
                            scales, (int32_t)pool.pages, indices, (int32_t)n_ind, indptr, last, op,
-                           static_cast<float*>(o.lse_ptr), causal, (float)scale, stream);
+                           static_cast<float*>(o.lse_ptr), causal, (float)scale, scratch.ptr,
+                           scratch.bytes, stream);
   Py_END_ALLOW_THREADS
   return rc ? PyLong_FromLong(rc) : o.result();
   END_HANDLE_TH_ERRORS
@@ -422,12 +438,10 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return p;
   };
   Entries e;
-  e.decode_run = reinterpret_cast<decltype(e.decode_run)>(at("pagedattn_decode_run"));
-  e.decode_run_append =
-      reinterpret_cast<decltype(e.decode_run_append)>(at("pagedattn_decode_run_append"));
-  e.decode_run_rope_append =
-      reinterpret_cast<decltype(e.decode_run_rope_append)>(at("pagedattn_decode_run_rope_append"));
-  e.prefill_run = reinterpret_cast<decltype(e.prefill_run)>(at("pagedattn_prefill_run"));
+  e.scratch_bytes =
+      reinterpret_cast<decltype(e.scratch_bytes)>(at("pagedattn_plan_scratch_bytes"));
+  e.decode_run = reinterpret_cast<decltype(e.decode_run)>(at("pagedattn_decode_run_scratch"));
+  e.prefill_run = reinterpret_cast<decltype(e.prefill_run)>(at("pagedattn_prefill_run_scratch"));
   e.append = reinterpret_cast<decltype(e.append)>(at("pagedattn_append_paged_kv_cache"));
   e.rope_append =
       reinterpret_cast<decltype(e.rope_append)>(at("pagedattn_rope_append_paged_kv_cache"));

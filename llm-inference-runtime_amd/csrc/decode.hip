@@ -1583,7 +1583,7 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
                            const int32_t* kv_indptr,
                            const int32_t* kv_last_page_len, void* out,
                            float* lse, float sm_scale, const AppendRows* app,
-                           void* stream) {
+                           void* stream, void* scratch = nullptr, size_t scratch_bytes = 0) {
   if (!plan || plan->mode != kPlanDecode)
     return set_error(PAGEDATTN_ERR_PLAN, "%s: no decode plan (call plan first)",
                      who);
@@ -1610,11 +1610,18 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
                      who);
   if (num_pages < 0 || num_indices < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: negative sizes", who);
+  // a plan of both forms runs its whole items where the run brings no scratch
+  const bool whole = plan->scratch_bytes && !scratch;
+  const bool own = plan->scratch_bytes && scratch;
+  if (own) {
+    const int rc = check_scratch(plan, who, scratch, scratch_bytes);
+    if (rc) return rc;
+  }
 
   DecodeParams p;
-  p.items = static_cast<const DecodeItem*>(plan->items_dev);
+  p.items = static_cast<const DecodeItem*>(whole ? plan->whole_dev : plan->items_dev);
   p.wave_ptr = plan->wave_ptr_dev;
-  p.n_groups = plan->n_items;
+  p.n_groups = whole ? plan->n_whole : plan->n_items;
   p.hg_shift = plan->hg_shift;
   p.deterministic = plan->deterministic ? 1 : 0;
   p.item_cost = plan->item_cost;
@@ -1633,8 +1640,9 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
   p.last_page_len = kv_last_page_len;
   p.out = static_cast<uint16_t*>(out);
   p.lse = lse;
-  p.partial_o = plan->partial_o;
-  p.partial_lse = plan->partial_lse;
+  p.partial_o = own ? static_cast<float*>(scratch) : plan->partial_o;
+  p.partial_lse = own ? reinterpret_cast<float*>(static_cast<char*>(scratch) + plan->scratch_lse)
+                      : plan->partial_lse;
   p.hq = plan->hq;
   p.hkv = plan->hkv;
   p.g = plan->hq / plan->hkv;
@@ -1654,7 +1662,7 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
 
   hipStream_t s = (hipStream_t)stream;
   const bool bf16 = q_dtype == PAGEDATTN_BF16;
-  if (plan->shared) {
+  if (plan->shared || whole) {
     // a device-planned shared plan (implicit) finds its items from kv_indptr,
     // unless pagedattn_decode_plan_device_update has dealt them into the
     // workspace (read as a host plan's)
@@ -1663,7 +1671,7 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
     if (!fn)
       return set_error(PAGEDATTN_ERR_UNSUPPORTED, "%s: shared-item plan for D = %d", who,
                        plan->d);
-    hipLaunchKernelGGL(fn, dim3(plan->n_items), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(fn, dim3(p.n_groups), dim3(256), 0, s, p);
     return check_launch(who);
   }
   DecodeFn fn = pick_decode(plan->d, bf16, fp8, app != nullptr, app && app->rope,
@@ -1694,8 +1702,8 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
                   : (bf16 ? decode_merge_kernel<true, 128> : decode_merge_kernel<false, 128>);
   hipLaunchKernelGGL(mfn, grid,
                      dim3(plan->max_pieces > kMergeClasses ? kWave * kMergeClasses : plan->d), 0, s,
-                     static_cast<const MergeItem*>(plan->merge_dev), plan->partial_o,
-                     plan->partial_lse, p.out, lse, plan->hq, p.g);
+                     static_cast<const MergeItem*>(plan->merge_dev), p.partial_o, p.partial_lse,
+                     p.out, lse, plan->hq, p.g);
   return check_launch("decode_run(merge)");
 }
 
@@ -1728,6 +1736,47 @@ int pagedattn_decode_plan_device_update(pagedattn_plan* plan, const int32_t* kv_
   return PAGEDATTN_OK;
 }
 
+int pagedattn_decode_run_scratch(
+    const pagedattn_plan* plan, const void* q, int64_t q_stride_n,
+    int64_t q_stride_h, int32_t q_dtype, const void* append_key,
+    const void* append_value, int64_t k_stride_n, int64_t k_stride_h,
+    int64_t v_stride_n, int64_t v_stride_h, int32_t rope,
+    const int32_t* positions, float rope_scale, float rope_theta,
+    void* paged_kv_cache, int32_t kv_dtype, const float* kv_scales,
+    int32_t num_pages, const int32_t* kv_indices, int32_t num_indices,
+    const int32_t* kv_indptr, const int32_t* kv_last_page_len, void* out,
+    float* lse, float sm_scale, void* scratch, size_t scratch_bytes, void* stream) {
+  const bool append = append_key || append_value;
+  const char* who = !append ? "decode_run" : rope ? "decode_run_rope_append" : "decode_run_append";
+  // skipped tokens are counted in the int32 at byte 0 of the workspace,
+  // clamped e4m3 pieces in the one at byte 4
+  AppendRows app{append_key, append_value, k_stride_n, k_stride_h, v_stride_n, v_stride_h,
+                 q_dtype, rope != 0, rope ? positions : nullptr, 1.0, 0.0,
+                 plan ? static_cast<int32_t*>(plan->workspace) : nullptr};
+  if (append) {
+    if (!append_key || !append_value)
+      return set_error(PAGEDATTN_ERR_INVALID, "%s: null append rows", who);
+    if ((k_stride_n & 7) || (k_stride_h & 7) || (v_stride_n & 7) ||
+        (v_stride_h & 7) || !aligned16(append_key) || !aligned16(append_value))
+      return set_error(PAGEDATTN_ERR_UNSUPPORTED,
+                       "%s: append rows must be 16-byte aligned with strides that "
+                       "are multiples of 8 elements",
+                       who);
+    if (rope) {
+      if (!(rope_scale > 0.f) || !(rope_theta > 0.f))
+        return set_error(PAGEDATTN_ERR_INVALID, "%s: rope_scale and rope_theta must be > 0",
+                         who);
+      app.rope_inv_scale = 1.0 / (double)rope_scale;
+      app.rope_log2_theta = std::log2((double)rope_theta);
+    }
+  }
+  return decode_run_impl(who, plan, q, q_stride_n, q_stride_h, q_dtype,
+                         paged_kv_cache, kv_dtype, kv_scales, num_pages,
+                         kv_indices, num_indices, kv_indptr, kv_last_page_len,
+                         out, lse, sm_scale, append ? &app : nullptr, stream, scratch,
+                         scratch_bytes);
+}
+
 int pagedattn_decode_run(const pagedattn_plan* plan, const void* q,
                          int64_t q_stride_n, int64_t q_stride_h,
                          int32_t q_dtype, const void* paged_kv_cache,
@@ -1751,24 +1800,13 @@ int pagedattn_decode_run_append(
     const int32_t* kv_indices, int32_t num_indices, const int32_t* kv_indptr,
     const int32_t* kv_last_page_len, void* out, float* lse, float sm_scale,
     void* stream) {
-  const char* who = "decode_run_append";
   if (!append_key || !append_value)
-    return set_error(PAGEDATTN_ERR_INVALID, "%s: null append rows", who);
-  if ((k_stride_n & 7) || (k_stride_h & 7) || (v_stride_n & 7) ||
-      (v_stride_h & 7) || !aligned16(append_key) || !aligned16(append_value))
-    return set_error(PAGEDATTN_ERR_UNSUPPORTED,
-                     "%s: append rows must be 16-byte aligned with strides that "
-                     "are multiples of 8 elements",
-                     who);
-  // skipped tokens are counted in the int32 at byte 0 of the workspace,
-  // clamped e4m3 pieces in the one at byte 4
-  AppendRows app{append_key, append_value, k_stride_n, k_stride_h,
-                 v_stride_n, v_stride_h, q_dtype, false, nullptr, 1.0, 0.0,
-                 plan ? static_cast<int32_t*>(plan->workspace) : nullptr};
-  return decode_run_impl(who, plan, q, q_stride_n, q_stride_h, q_dtype,
-                         paged_kv_cache, kv_dtype, kv_scales, num_pages,
-                         kv_indices, num_indices, kv_indptr, kv_last_page_len,
-                         out, lse, sm_scale, &app, stream);
+    return set_error(PAGEDATTN_ERR_INVALID, "decode_run_append: null append rows");
+  return pagedattn_decode_run_scratch(
+      plan, q, q_stride_n, q_stride_h, q_dtype, append_key, append_value, k_stride_n, k_stride_h,
+      v_stride_n, v_stride_h, 0, nullptr, 1.f, 1.f, paged_kv_cache, kv_dtype, kv_scales,
+      num_pages, kv_indices, num_indices, kv_indptr, kv_last_page_len, out, lse, sm_scale,
+      nullptr, 0, stream);
 }
 
 int pagedattn_decode_run_rope_append(
@@ -1781,26 +1819,13 @@ int pagedattn_decode_run_rope_append(
     int32_t num_indices, const int32_t* kv_indptr,
     const int32_t* kv_last_page_len, void* out, float* lse, float sm_scale,
     void* stream) {
-  const char* who = "decode_run_rope_append";
   if (!append_key || !append_value)
-    return set_error(PAGEDATTN_ERR_INVALID, "%s: null append rows", who);
-  if ((k_stride_n & 7) || (k_stride_h & 7) || (v_stride_n & 7) ||
-      (v_stride_h & 7) || !aligned16(append_key) || !aligned16(append_value))
-    return set_error(PAGEDATTN_ERR_UNSUPPORTED,
-                     "%s: append rows must be 16-byte aligned with strides that "
-                     "are multiples of 8 elements",
-                     who);
-  if (!(rope_scale > 0.f) || !(rope_theta > 0.f))
-    return set_error(PAGEDATTN_ERR_INVALID, "%s: rope_scale and rope_theta must be > 0",
-                     who);
-  AppendRows app{append_key, append_value, k_stride_n, k_stride_h, v_stride_n,
-                 v_stride_h, q_dtype, true, positions, 1.0 / (double)rope_scale,
-                 std::log2((double)rope_theta),
-                 plan ? static_cast<int32_t*>(plan->workspace) : nullptr};
-  return decode_run_impl(who, plan, q, q_stride_n, q_stride_h, q_dtype,
-                         paged_kv_cache, kv_dtype, kv_scales, num_pages,
-                         kv_indices, num_indices, kv_indptr, kv_last_page_len,
-                         out, lse, sm_scale, &app, stream);
+    return set_error(PAGEDATTN_ERR_INVALID, "decode_run_rope_append: null append rows");
+  return pagedattn_decode_run_scratch(
+      plan, q, q_stride_n, q_stride_h, q_dtype, append_key, append_value, k_stride_n, k_stride_h,
+      v_stride_n, v_stride_h, 1, positions, rope_scale, rope_theta, paged_kv_cache, kv_dtype,
+      kv_scales, num_pages, kv_indices, num_indices, kv_indptr, kv_last_page_len, out, lse,
+      sm_scale, nullptr, 0, stream);
 }
 
 }  // extern "C"

@@ -362,6 +362,7 @@ int setup_device_plan(const char* who, pagedattn_plan* plan, int32_t batch_size,
                              int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,
                              int32_t page_size, int cus, char* partials, size_t bytes) {
   plan->mode = kPlanNone;
+  plan->scratch_bytes = 0;
   if (batch_size < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: batch_size %d < 0", who, batch_size);
   int rc = validate_heads(who, num_qo_heads, num_kv_heads, head_dim, page_size);
@@ -416,6 +417,7 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
   const char* who = "decode_plan";
   if (!plan) return set_error(PAGEDATTN_ERR_INVALID, "%s: null plan", who);
   plan->mode = kPlanNone;
+  plan->scratch_bytes = 0;
   if (batch_size < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: batch_size %d < 0", who,
                      batch_size);
@@ -635,9 +637,14 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
   const size_t off_pl =
       ws_align(off_po + sizeof(float) * (size_t)n_slots * g * head_dim);
   const size_t end = ws_align(off_pl + sizeof(float) * (size_t)n_slots * g);
-  const size_t host_bytes = off_po - kWsHeader;
-  // a small batch whose partials do not fit stays whole
-  if (fit == kSharedFallback && end > workspace_bytes) return use_shared();
+  // a small batch that is faster cut keeps the whole items beside the cut list:
+  // its runs bring their own scratch for the partials, or run the whole items.
+  // Where the workspace could not hold the partials, or both lists, it is not cut.
+  const bool both = fit == kSharedFallback && n_slots > 0;
+  const size_t whole_end = ws_align(off_po + sizeof(SharedItem) * sitems.size());
+  if (fit == kSharedFallback && (both ? std::max(end, whole_end) : end) > workspace_bytes)
+    return use_shared();
+  const size_t host_bytes = (both ? whole_end : off_po) - kWsHeader;
 
   plan->host.assign(host_bytes / sizeof(int32_t), 0);
   char* hb = reinterpret_cast<char*>(plan->host.data());
@@ -646,10 +653,12 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
   std::memcpy(hb + (off_wave - kWsHeader), wave_ptr.data(), sizeof(int32_t) * (n_waves + 1));
   if (n_merge)
     std::memcpy(hb + (off_merge - kWsHeader), merges.data(), sizeof(MergeItem) * n_merge);
+  if (both)
+    std::memcpy(hb + (off_po - kWsHeader), sitems.data(), sizeof(SharedItem) * sitems.size());
 
   plan->workspace = workspace;
   plan->workspace_bytes = workspace_bytes;
-  rc = upload_plan(plan, who, host_bytes, end, stream);
+  rc = upload_plan(plan, who, host_bytes, both ? whole_end : end, stream);
   if (rc) return rc;
 
   char* ws = static_cast<char*>(workspace);
@@ -668,8 +677,14 @@ int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
   plan->items_dev = ws + off_items;
   plan->wave_ptr_dev = reinterpret_cast<const int32_t*>(ws + off_wave);
   plan->merge_dev = ws + off_merge;
-  plan->partial_o = reinterpret_cast<float*>(ws + off_po);
-  plan->partial_lse = reinterpret_cast<float*>(ws + off_pl);
+  plan->partial_o = both ? nullptr : reinterpret_cast<float*>(ws + off_po);
+  plan->partial_lse = both ? nullptr : reinterpret_cast<float*>(ws + off_pl);
+  if (both) {
+    plan->whole_dev = ws + off_po;
+    plan->n_whole = n_wg;
+    plan->deterministic = decode_deterministic();
+    plan->scratch_bytes = partial_bytes((int64_t)n_slots * g, head_dim, &plan->scratch_lse);
+  }
   plan->total_pages = total;
   plan->max_pages = maxp;
   plan->mode = kPlanDecode;

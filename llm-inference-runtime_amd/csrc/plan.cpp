@@ -81,6 +81,16 @@ int upload_plan(pagedattn_plan* plan, const char* who, size_t host_bytes,
   return PAGEDATTN_OK;
 }
 
+int check_scratch(const pagedattn_plan* plan, const char* who, const void* scratch,
+                  size_t scratch_bytes) {
+  if ((uintptr_t)scratch & (kWsAlign - 1))
+    return set_error(PAGEDATTN_ERR_INVALID, "%s: the scratch must be 256-byte aligned", who);
+  if (scratch_bytes < plan->scratch_bytes)
+    return set_error(PAGEDATTN_ERR_WORKSPACE, "%s: needs %zu scratch bytes, %zu given", who,
+                     plan->scratch_bytes, scratch_bytes);
+  return PAGEDATTN_OK;
+}
+
 }  // namespace pa
 
 extern "C" {
@@ -88,5 +98,9 @@ extern "C" {
 pagedattn_plan* pagedattn_plan_create(void) { return new pagedattn_plan(); }
 
 void pagedattn_plan_destroy(pagedattn_plan* plan) { delete plan; }
+
+size_t pagedattn_plan_scratch_bytes(const pagedattn_plan* plan) {
+  return plan && plan->mode != pa::kPlanNone ? plan->scratch_bytes : 0;
+}
 
 }  // extern "C"

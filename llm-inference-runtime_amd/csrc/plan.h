@@ -113,11 +113,11 @@ inline __host__ __device__ bool prefill_split_pays(int t_max, int len, int64_t c
   return t_max - len >= 4 && cost < 3 * slots * t_max;
 }
 
-// Workspace of a split prefill plan, from the workspace start: the cut tiles'
-// count, `entries` work-list entries, the merge list and the partials of
-// `slots` slots of every KV head.
+// Workspace of a prefill plan that may cut tiles, from the workspace start: the
+// `tiles` whole tiles, the cut tiles' count, `entries` pieces and the merge list
+// of at most `slots` pieces per KV head.
 struct PrefillSplitLayout {
-  size_t off_count, off_pieces, off_merges, off_po, off_pl, end;
+  size_t off_items, off_count, off_pieces, off_merges, end;
 };
 
 // Workspace layout: [0, kWsHeader) is reserved for the caller's device flags
@@ -127,16 +127,21 @@ constexpr size_t kWsAlign = 256;
 
 inline size_t ws_align(size_t x) { return (x + kWsAlign - 1) & ~(kWsAlign - 1); }
 
-inline PrefillSplitLayout prefill_split_layout(int64_t entries, int64_t slots, int hkv, int d) {
+inline PrefillSplitLayout prefill_split_layout(int64_t tiles, int64_t entries, int64_t slots) {
   PrefillSplitLayout l;
-  l.off_count = kWsHeader;
+  l.off_items = kWsHeader;
+  l.off_count = ws_align(l.off_items + sizeof(PrefillItem) * (size_t)tiles);
   l.off_pieces = l.off_count + kWsAlign;
   l.off_merges = ws_align(l.off_pieces + sizeof(PrefillPiece) * (size_t)entries);
-  l.off_po = ws_align(l.off_merges + sizeof(PrefillMerge) * (size_t)(slots / 2 + 1));
-  const size_t rows = (size_t)slots * hkv * kPrefillRows;
-  l.off_pl = ws_align(l.off_po + sizeof(float) * rows * d);
-  l.end = ws_align(l.off_pl + sizeof(float) * rows);
+  l.end = ws_align(l.off_merges + sizeof(PrefillMerge) * (size_t)(slots / 2 + 1));
   return l;
+}
+
+// A run's split partials: outputs of `rows` rows of d values, then from *off_lse
+// their log-sum-exps.  Returns the bytes of both.
+inline size_t partial_bytes(int64_t rows, int d, size_t* off_lse) {
+  *off_lse = ws_align(sizeof(float) * (size_t)rows * d);
+  return ws_align(*off_lse + sizeof(float) * (size_t)rows);
 }
 
 }  // namespace pa
@@ -174,12 +179,22 @@ struct pagedattn_plan {
   // prefill: tiles of at most half a workgroup's rows run as KV-head pairs
   // (device plans apply it at run time; host plans flag their items)
   bool prefill_pair = false;
-  // prefill: the work list is one of PrefillPiece entries with a merge list
-  // and n_slots partial slots per KV head (host plans: some tile is cut;
-  // device plans: the plan kernel may cut tiles)
-  bool prefill_split = false;
-  int q_cap = 0;  // device plans that may cut tiles: q-tiles the plan holds
   int64_t total_qo = 0;
+  // > 0: the plan holds two work lists, one that cuts KV ranges and a whole one
+  // that writes nothing but the outputs.  A run that brings this many bytes of
+  // scratch for its split partials takes the cut list, any other the whole one,
+  // so runs of one plan share no memory that they write and may overlap.
+  // prefill: items_dev is the whole list, pieces_dev / merge_dev the cut one
+  // with n_slots slots per KV head (device plans: the plan kernel writes both).
+  // decode: items_dev / merge_dev are the cut list, whole_dev the shared items
+  // of n_whole workgroups.
+  size_t scratch_bytes = 0;
+  size_t scratch_lse = 0;  // offset of the partial log-sum-exps in the scratch
+  int n_pieces = 0;
+  void* pieces_dev = nullptr;
+  int32_t* n_merge_dev = nullptr;  // prefill: the cut tiles' count
+  int n_whole = 0;
+  void* whole_dev = nullptr;
   // device pointers into the workspace
   void* items_dev = nullptr;
   const int32_t* wave_ptr_dev = nullptr;  // decode: items of head group w

@@ -24,6 +24,11 @@ int validate_heads(const char* who, int32_t hq, int32_t hkv, int32_t d,
 int upload_plan(pagedattn_plan* plan, const char* who, size_t host_bytes,
                 size_t total_bytes, void* stream);
 
+// Checks the scratch a run brings for a plan's split partials (256-byte
+// aligned, at least plan->scratch_bytes).
+int check_scratch(const pagedattn_plan* plan, const char* who, const void* scratch,
+                  size_t scratch_bytes);
+
 // The device-side partition of a decode plan (pagedattn_decode_plan_device
 // and pagedattn_decode_run_noalloc): shares of the (sequence, head group,
 // page) stream for cus x waves-per-CU / hg head groups, split partials at

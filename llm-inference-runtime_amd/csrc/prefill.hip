@@ -42,7 +42,7 @@
 namespace pa {
 
 struct PrefillParams {
-  const PrefillItem* items;  // SPLIT: PrefillPiece entries
+  const PrefillItem* items;  // SPLIT: PrefillPiece entries (n_items of them)
   int32_t n_items, batch_size;
   const uint16_t* q;
   int64_t q_sn, q_sh;
@@ -863,9 +863,9 @@ static PrefillFn pick_prefill(int d, bool bf16, bool fp8, bool split) {
 // tile's output is the same wherever it runs.  Entries past the tiles, up to
 // the plan's capacity, get b = -1 (the attention workgroups return at once);
 // tiles beyond the capacity are dropped and counted in `dropped`.
-// Plans with `slots` > 0 write PrefillPiece entries and cut long tiles of a
-// small step by the host planner's rule (plan.h): 8 threads count the pieces
-// of each of the 128 candidate cuts.
+// Plans with `slots` > 0 also write the list of pieces, in which long tiles of a
+// small step are cut by the host planner's rule (plan.h): 8 threads count the
+// pieces of each of the 128 candidate cuts.
 struct PrefillPlanArgs {
   const int32_t* qo_indptr;
   const int32_t* kv_indptr;
@@ -946,13 +946,10 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
     const int flag = a.pair && (int64_t)(q_hi - q_lo) * a.g <= kPrefillRows / 2 ? 1 : -1;
     return PrefillItem{b, q_lo, q_hi, flag};
   };
-  auto put = [&](int at, const PrefillItem& it) {
-    if (a.slots > 0)
-      a.pieces[at] = PrefillPiece{it.b, it.q_lo, it.q_hi, it.slot, 0, 1, -1, 0};
-    else
-      a.items[at] = it;
+  auto put_piece = [&](int at, const PrefillItem& it) {
+    if (a.slots > 0) a.pieces[at] = PrefillPiece{it.b, it.q_lo, it.q_hi, it.slot, 0, 1, -1, 0};
   };
-  int used = n_tiles;  // list entries written
+  int used = n_tiles;  // pieces written
   int n_merge = 0;
   if (n_tiles <= kPrefillDevSortMax) {
     // one tile per thread; its rank among unique keys (cost, then sequence
@@ -1026,47 +1023,47 @@ __global__ void __launch_bounds__(kPrefillPlanThreads) prefill_plan_kernel(Prefi
           a.merges[(int)(key[rank] & 0x7fffffff)] =
               PrefillMerge{it.b, it.q_lo, it.q_hi, at, n, 0, 0, 0};
       }
-    } else if (t < n_tiles) {
+    }
+    if (t < n_tiles) {
       // paired tiles alternate between the even and the odd head of a head
       // pair by list position, so both XCDs of the pair share them
       if (it.slot > 0) it.slot = 1 + (rank & 1);
-      put(rank, it);
+      a.items[rank] = it;
+      if (len == 0) put_piece(rank, it);
     }
   } else {
     for (int i = t; i < n_tiles; i += kPrefillPlanThreads) {
       PrefillItem it = tile(i, nullptr);
       if (it.slot > 0) it.slot = 1 + (i & 1);
-      put(i, it);
+      a.items[i] = it;
+      put_piece(i, it);
     }
   }
-  if (a.slots > 0 && t == 0) *a.n_merge = n_merge;
-  const int end = a.slots > 0 ? a.entries : a.cap;
-  for (int i = used + t; i < end; i += kPrefillPlanThreads) put(i, PrefillItem{-1, 0, 0, -1});
+  for (int i = n_tiles + t; i < a.cap; i += kPrefillPlanThreads)
+    a.items[i] = PrefillItem{-1, 0, 0, -1};
+  if (a.slots > 0) {
+    if (t == 0) *a.n_merge = n_merge;
+    for (int i = used + t; i < a.entries; i += kPrefillPlanThreads)
+      put_piece(i, PrefillItem{-1, 0, 0, -1});
+  }
 }
 
 }  // namespace pa
 
 namespace pa {
 
-// The cut tiles' count of a split plan's merge list.
-static int32_t* split_count(const pagedattn_plan* plan) {
-  return reinterpret_cast<int32_t*>(static_cast<char*>(plan->workspace) + kWsHeader);
-}
-
 // The q-tile list of a device prefill plan, cut from the metadata on the
 // device by one workgroup (prefill_plan_kernel) on `stream`.
 static int launch_prefill_plan(const pagedattn_plan* plan, const int32_t* qo_indptr,
                                const int32_t* kv_indptr, const int32_t* kv_last_page_len,
                                void* stream, const char* who) {
-  const bool split = plan->prefill_split;
   PrefillPlanArgs a{qo_indptr, kv_indptr, kv_last_page_len, plan->batch_size,
                     plan->q_tile, plan->hq / plan->hkv, plan->prefill_pair ? 1 : 0,
-                    split ? plan->q_cap : plan->n_items,
-                    static_cast<PrefillItem*>(plan->items_dev),
+                    plan->n_items, static_cast<PrefillItem*>(plan->items_dev),
                     reinterpret_cast<int32_t*>(static_cast<char*>(plan->workspace) + 12),
-                    split ? plan->n_slots : 0, plan->n_items,
-                    static_cast<PrefillPiece*>(plan->items_dev),
-                    static_cast<PrefillMerge*>(plan->merge_dev), split_count(plan)};
+                    plan->scratch_bytes ? plan->n_slots : 0, plan->n_pieces,
+                    static_cast<PrefillPiece*>(plan->pieces_dev),
+                    static_cast<PrefillMerge*>(plan->merge_dev), plan->n_merge_dev};
   hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPrefillPlanThreads), 0,
                      (hipStream_t)stream, a);
   return check_launch(who);
@@ -1110,6 +1107,22 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
                           const int32_t* kv_last_page_len, void* out,
                           float* lse, int32_t causal, float sm_scale,
                           void* stream) {
+  return pagedattn_prefill_run_scratch(plan, q, q_stride_n, q_stride_h, q_dtype, qo_indptr,
+                                       paged_kv_cache, kv_dtype, kv_scales, num_pages, kv_indices,
+                                       num_indices, kv_indptr, kv_last_page_len, out, lse, causal,
+                                       sm_scale, nullptr, 0, stream);
+}
+
+int pagedattn_prefill_run_scratch(const pagedattn_plan* plan, const void* q,
+                                  int64_t q_stride_n, int64_t q_stride_h,
+                                  int32_t q_dtype, const int32_t* qo_indptr,
+                                  const void* paged_kv_cache, int32_t kv_dtype,
+                                  const float* kv_scales, int32_t num_pages,
+                                  const int32_t* kv_indices, int32_t num_indices,
+                                  const int32_t* kv_indptr,
+                                  const int32_t* kv_last_page_len, void* out,
+                                  float* lse, int32_t causal, float sm_scale,
+                                  void* scratch, size_t scratch_bytes, void* stream) {
   const char* who = "prefill_run";
   if (!plan || plan->mode != kPlanPrefill)
     return set_error(PAGEDATTN_ERR_PLAN,
@@ -1134,6 +1147,11 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
                      plan->batch_size);
   if ((int64_t)plan->n_items * plan->hkv > INT32_MAX)
     return set_error(PAGEDATTN_ERR_UNSUPPORTED, "%s: too many work items", who);
+  const bool cut = plan->scratch_bytes && scratch;
+  if (cut) {
+    const int rc = check_scratch(plan, who, scratch, scratch_bytes);
+    if (rc) return rc;
+  }
   if (!q || !qo_indptr || !paged_kv_cache || !kv_indices || !kv_indptr ||
       !kv_last_page_len || !out)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: null pointer", who);
@@ -1146,8 +1164,8 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   if (num_pages < 0 || num_indices < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: negative sizes", who);
   PrefillParams p;
-  p.items = static_cast<const PrefillItem*>(plan->items_dev);
-  p.n_items = plan->n_items;
+  p.items = static_cast<const PrefillItem*>(cut ? plan->pieces_dev : plan->items_dev);
+  p.n_items = cut ? plan->n_pieces : plan->n_items;
   p.batch_size = plan->batch_size;
   p.q = static_cast<const uint16_t*>(q);
   p.q_sn = q_stride_n;
@@ -1167,28 +1185,29 @@ int pagedattn_prefill_run(const pagedattn_plan* plan, const void* q,
   p.g = plan->hq / plan->hkv;
   p.causal = causal ? 1 : 0;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
-  p.partial_o = plan->partial_o;
-  p.partial_lse = plan->partial_lse;
-  p.n_slots = plan->n_slots;
+  p.partial_o = cut ? static_cast<float*>(scratch) : nullptr;
+  p.partial_lse =
+      cut ? reinterpret_cast<float*>(static_cast<char*>(scratch) + plan->scratch_lse) : nullptr;
+  p.n_slots = cut ? plan->n_slots : 0;
   const bool bf16 = q_dtype == PAGEDATTN_BF16;
-  PrefillFn fn = pick_prefill(plan->d, bf16, fp8, plan->prefill_split);
+  PrefillFn fn = pick_prefill(plan->d, bf16, fp8, cut);
   if (plan->implicit && !plan->dev_table) {
     // the work list of this run, built on the device ahead of the attention
     // (unless pagedattn_prefill_plan_device_update built it for the step)
     int rc = launch_prefill_plan(plan, qo_indptr, kv_indptr, kv_last_page_len, stream, who);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(fn, dim3(plan->n_items * plan->hkv), dim3(64 * kPrefillWaves), 0,
+  hipLaunchKernelGGL(fn, dim3(p.n_items * plan->hkv), dim3(64 * kPrefillWaves), 0,
                      (hipStream_t)stream, p);
   const int rc = check_launch(who);
-  if (rc || !plan->prefill_split) return rc;
+  if (rc || !cut) return rc;
   // host plans know their cut tiles; a device plan's are at most half its
   // slots, and its merge workgroups find out how many there are
   const int cap = plan->implicit ? plan->n_slots / 2 : plan->n_merge;
   PrefillMergeArgs m{static_cast<const PrefillMerge*>(plan->merge_dev),
-                     plan->implicit ? split_count(plan) : nullptr, cap,
+                     plan->implicit ? plan->n_merge_dev : nullptr, cap,
                      plan->batch_size, plan->hq, plan->hkv, p.g, plan->n_slots, qo_indptr,
-                     plan->partial_o, plan->partial_lse, p.out, lse};
+                     p.partial_o, p.partial_lse, p.out, lse};
   const int64_t units = (int64_t)cap * (kPrefillRows / 32) * (plan->d / 32) * plan->hkv;
   auto* mfn = plan->d == 64
                   ? (bf16 ? prefill_merge_kernel<true, 64> : prefill_merge_kernel<false, 64>)

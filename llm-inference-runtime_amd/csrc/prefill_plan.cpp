@@ -61,15 +61,32 @@ static int prefill_piece_tiles(const std::vector<int>& tiles, int64_t slots) {
   return best > 0 && prefill_split_pays(t_max, best, best_cost, slots) ? best : 0;
 }
 
-// The device side of a split plan: work list, merge list and partials.
-static void set_split(pagedattn_plan* plan, const PrefillSplitLayout& lay, int64_t slots) {
+// Rows of split partials of `slots` pieces per KV head.
+static int64_t prefill_partial_rows(int64_t slots, int hkv) {
+  return slots * hkv * kPrefillRows;
+}
+
+// Whether plans may cut tiles: the caller's workspace bounds the scratch that
+// their runs ask for (the same bound for host and device plans, whose outputs
+// then agree bit for bit).
+static bool prefill_may_cut(int64_t slots, int hkv, int d, size_t workspace_bytes) {
+  size_t off_lse;
+  return prefill_splitting() && slots >= 2 &&
+         kWsHeader + partial_bytes(prefill_partial_rows(slots, hkv), d, &off_lse) <=
+             workspace_bytes;
+}
+
+// The cut list of a plan: n_pieces entries over `slots` slots per KV head.
+static void set_split(pagedattn_plan* plan, const PrefillSplitLayout& lay, int64_t n_pieces,
+                      int64_t slots) {
   char* ws = static_cast<char*>(plan->workspace);
-  plan->prefill_split = true;
+  plan->n_pieces = (int)n_pieces;
   plan->n_slots = (int)slots;
-  plan->items_dev = ws + lay.off_pieces;
+  plan->pieces_dev = ws + lay.off_pieces;
   plan->merge_dev = ws + lay.off_merges;
-  plan->partial_o = reinterpret_cast<float*>(ws + lay.off_po);
-  plan->partial_lse = reinterpret_cast<float*>(ws + lay.off_pl);
+  plan->n_merge_dev = reinterpret_cast<int32_t*>(ws + lay.off_count);
+  plan->scratch_bytes = partial_bytes(prefill_partial_rows(slots, plan->hkv), plan->d,
+                                      &plan->scratch_lse);
 }
 
 }  // namespace pa
@@ -88,6 +105,7 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
   const char* who = "prefill_plan";
   if (!plan) return set_error(PAGEDATTN_ERR_INVALID, "%s: null plan", who);
   plan->mode = kPlanNone;
+  plan->scratch_bytes = 0;
   if (batch_size < 0)
     return set_error(PAGEDATTN_ERR_INVALID, "%s: batch_size %d < 0", who,
                      batch_size);
@@ -159,18 +177,17 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
   std::stable_sort(order.begin(), order.end(),
                    [&](int a, int c) { return cost[a] > cost[c]; });
-  plan->prefill_split = false;
   const int64_t slots = prefill_split_slots(num_kv_heads);
-  const PrefillSplitLayout lay = prefill_split_layout(slots, slots, num_kv_heads, head_dim);
   int piece_tiles = 0;
-  if (prefill_splitting() && lay.end <= workspace_bytes && (int64_t)items.size() <= slots) {
+  if (prefill_may_cut(slots, num_kv_heads, head_dim, workspace_bytes) &&
+      (int64_t)items.size() <= slots) {
     std::vector<int> tiles;
     for (int64_t c : cost) tiles.push_back((int)((c + kPrefillKvTile - 1) / kPrefillKvTile));
     piece_tiles = prefill_piece_tiles(tiles, slots);
   }
-  if (piece_tiles > 0) {
-    std::vector<PrefillPiece> pieces;
-    std::vector<PrefillMerge> merges;
+  std::vector<PrefillPiece> pieces;
+  std::vector<PrefillMerge> merges;
+  if (piece_tiles > 0)
     for (int i : order) {
       const PrefillItem& it = items[i];
       const int t = (int)((cost[i] + kPrefillKvTile - 1) / kPrefillKvTile);
@@ -180,28 +197,21 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
         pieces.push_back(PrefillPiece{it.b, it.q_lo, it.q_hi, -1, k, n, n > 1 ? at + k : -1, 0});
       if (n > 1) merges.push_back(PrefillMerge{it.b, it.q_lo, it.q_hi, at, n, 0, 0, 0});
     }
-    const size_t host_bytes = lay.off_po - kWsHeader;
-    plan->host.assign(host_bytes / sizeof(int32_t), 0);
-    char* hb = reinterpret_cast<char*>(plan->host.data());
+  const bool cut = !merges.empty();
+  const PrefillSplitLayout lay = prefill_split_layout(n_tiles, (int64_t)pieces.size(), slots);
+  const size_t host_bytes =
+      cut ? lay.end - kWsHeader : sizeof(PrefillItem) * items.size();
+  plan->host.assign((host_bytes + 3) / 4, 0);
+  char* hb = reinterpret_cast<char*>(plan->host.data());
+  if (cut) {
     const int32_t n_merge = (int32_t)merges.size();
     std::memcpy(hb + (lay.off_count - kWsHeader), &n_merge, sizeof(n_merge));
     std::memcpy(hb + (lay.off_pieces - kWsHeader), pieces.data(),
                 sizeof(PrefillPiece) * pieces.size());
     std::memcpy(hb + (lay.off_merges - kWsHeader), merges.data(),
                 sizeof(PrefillMerge) * merges.size());
-    plan->workspace = workspace;
-    plan->workspace_bytes = workspace_bytes;
-    rc = upload_plan(plan, who, host_bytes, lay.end, stream);
-    if (rc) return rc;
-    plan->n_items = (int)pieces.size();
-    plan->n_merge = n_merge;
-    set_split(plan, lay, slots);
-    finish(plan);
-    return PAGEDATTN_OK;
   }
-  const size_t host_bytes = sizeof(PrefillItem) * items.size();
-  plan->host.assign((host_bytes + 3) / 4, 0);
-  auto* dst = reinterpret_cast<PrefillItem*>(plan->host.data());
+  auto* dst = reinterpret_cast<PrefillItem*>(hb);
   // paired tiles alternate between the even and the odd head of each pair in
   // list order, so the two XCDs that hold a head pair's workgroups share them
   int n_paired = 0;
@@ -215,10 +225,11 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
                    stream);
   if (rc) return rc;
   plan->n_items = (int)items.size();
-  plan->n_merge = 0;
+  plan->n_merge = (int)merges.size();
   plan->n_slots = 0;
   plan->items_dev = static_cast<char*>(workspace) + kWsHeader;
   finish(plan);
+  if (cut) set_split(plan, lay, (int64_t)pieces.size(), (int64_t)pieces.size());
   return PAGEDATTN_OK;
 }
 
@@ -229,6 +240,7 @@ int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,
   const char* who = "prefill_plan_device";
   if (!plan) return set_error(PAGEDATTN_ERR_INVALID, "%s: null plan", who);
   plan->mode = kPlanNone;
+  plan->scratch_bytes = 0;
   if (batch_size < 0 || batch_size > kPrefillDevMaxBatch)
     return set_error(PAGEDATTN_ERR_UNSUPPORTED, "%s: batch_size %d outside [0, %d]", who,
                      batch_size, kPrefillDevMaxBatch);
@@ -267,18 +279,15 @@ int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,
   plan->q_tile = q_tile;
   plan->total_qo = max_qo_tokens;
   plan->items_dev = static_cast<char*>(workspace) + kWsHeader;
-  // a plan whose workspace holds the partials may cut tiles, on the host
-  // plan's rule (the tiles are known to the plan kernel only)
-  plan->prefill_split = false;
+  // the plan kernel may cut tiles, on the host plan's rule (the tiles are known
+  // to it only), where both lists fit
   const int64_t slots = prefill_split_slots(num_kv_heads);
   const int64_t entries = std::max(cap, slots);
-  const PrefillSplitLayout lay = prefill_split_layout(entries, slots, num_kv_heads, head_dim);
-  if (cap > 0 && prefill_splitting() && slots >= 2 && slots <= kPrefillDevSortMax &&
-      lay.end <= workspace_bytes && entries * num_kv_heads <= INT32_MAX) {
-    plan->n_items = (int)entries;
-    plan->q_cap = (int)cap;
-    set_split(plan, lay, slots);
-  }
+  const PrefillSplitLayout lay = prefill_split_layout(cap, entries, slots);
+  if (cap > 0 && prefill_may_cut(slots, num_kv_heads, head_dim, workspace_bytes) &&
+      slots <= kPrefillDevSortMax && lay.end <= workspace_bytes &&
+      entries * num_kv_heads <= INT32_MAX)
+    set_split(plan, lay, entries, slots);
   plan->mode = kPlanPrefill;
   return PAGEDATTN_OK;
 }

@@ -92,6 +92,12 @@ _SIGNATURES = {
         [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
          _c_p, _c_f, _c_f, _c_p, _c_int, _c_p, _c_int, _c_p, _c_int, _c_p, _c_p, _c_p, _c_p,
          _c_f, _c_p]),
+    "pagedattn_plan_scratch_bytes": (_c_sz, [_c_p]),
+    "pagedattn_decode_run_scratch": (
+        _c_int,
+        [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
+         _c_int, _c_p, _c_f, _c_f, _c_p, _c_int, _c_p, _c_int, _c_p, _c_int, _c_p, _c_p, _c_p,
+         _c_p, _c_f, _c_p, _c_sz, _c_p]),
     "pagedattn_decode_plan_device": (
         _c_int, [_c_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_p, _c_sz]),
     "pagedattn_decode_plan_device_update": (_c_int, [_c_p, _c_p, _c_p, _c_p]),
@@ -111,6 +117,10 @@ _SIGNATURES = {
         _c_int,
         [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_int, _c_p, _c_int,
          _c_p, _c_int, _c_p, _c_p, _c_p, _c_p, _c_int, _c_f, _c_p]),
+    "pagedattn_prefill_run_scratch": (
+        _c_int,
+        [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_int, _c_p, _c_int,
+         _c_p, _c_int, _c_p, _c_p, _c_p, _c_p, _c_int, _c_f, _c_p, _c_sz, _c_p]),
     "pagedattn_quantize_pages_e4m3": (
         _c_int, [_c_p, _c_int, _c_p, _c_p, _c_int, _c_int, _c_int, _c_int, _c_p]),
     "pagedattn_copy_bytes": (_c_int, [_c_p, _c_p, _c_sz, _c_p]),

@@ -114,6 +114,29 @@ def _native(fn: str, entry: str, *args):
     return r
 
 
+def _scratch(plan: "_Plan", device: torch.device) -> torch.Tensor | None:
+    """One run's scratch for the partials of a plan that cuts KV ranges, from
+    torch's caching allocator (per run and stream: runs of one plan may
+    overlap); None where the plan needs none, or where there is no memory for it
+    and the run takes the plan's whole form."""
+    n = _lib.lib().pagedattn_plan_scratch_bytes(plan.handle)
+    if n == 0:
+        return None
+    try:
+        return torch.empty(n, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def _run_plan(entry: str, fn: str, scratch: torch.Tensor | None, device: torch.device,
+              *args) -> None:
+    """Entry point `fn` with its scratch and stream arguments; errors name `entry`."""
+    rc = getattr(_lib.lib(), fn)(*args, ptr(scratch), 0 if scratch is None else scratch.numel(),
+                                 _stream(device))
+    if rc != 0:
+        _lib.raise_status(entry, rc)
+
+
 def _check_rows(x: torch.Tensor, name: str, heads: int | None, d: int | None):
     _require_cuda(x, name)
     if x.dim() != 3:
@@ -744,10 +767,9 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
             lse = torch.empty((self._bsz, self._hq), dtype=torch.float32, device=q.device)
         common = (ptr(paged_kv_cache), dtype_code(paged_kv_cache.dtype), ptr(scales),
                   num_pages, ptr(self._indices), self._indices.numel(), ptr(self._indptr),
-                  ptr(self._last), ptr(out), ptr(lse), float(scale), _stream(q.device))
+                  ptr(self._last), ptr(out), ptr(lse), float(scale))
         if append_key is None and append_value is None:
-            call("pagedattn_decode_run", self._plan.handle, ptr(q), q.stride(0), q.stride(1),
-                 dtype_code(q.dtype), *common)
+            rows = (None, None, 0, 0, 0, 0, 0, None, 1.0, 1.0)
         else:
             if append_key is None or append_value is None:
                 raise ValueError("append_key and append_value go together")
@@ -758,10 +780,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
             if rope is None:
                 if positions is not None:
                     raise ValueError("positions only applies together with rope")
-                call("pagedattn_decode_run_append", self._plan.handle, ptr(q), q.stride(0),
-                     q.stride(1), dtype_code(q.dtype), ptr(append_key), ptr(append_value),
-                     append_key.stride(0), append_key.stride(1), append_value.stride(0),
-                     append_value.stride(1), *common)
+                rotate = (0, None, 1.0, 1.0)
             else:
                 rope_scale, rope_theta = rope
                 pos = None
@@ -769,11 +788,13 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
                     if positions.numel() != self._bsz:
                         raise ValueError("positions must hold one entry per sequence")
                     pos = _i32(positions, q.device)
-                call("pagedattn_decode_run_rope_append", self._plan.handle, ptr(q),
-                     q.stride(0), q.stride(1), dtype_code(q.dtype), ptr(append_key),
-                     ptr(append_value), append_key.stride(0), append_key.stride(1),
-                     append_value.stride(0), append_value.stride(1), ptr(pos),
-                     float(rope_scale), float(rope_theta), *common)
+                rotate = (1, ptr(pos), float(rope_scale), float(rope_theta))
+            rows = (ptr(append_key), ptr(append_value), append_key.stride(0),
+                    append_key.stride(1), append_value.stride(0), append_value.stride(1),
+                    *rotate)
+        _run_plan(entry, "pagedattn_decode_run_scratch", _scratch(self._plan, q.device), q.device,
+                  self._plan.handle, ptr(q), q.stride(0), q.stride(1), dtype_code(q.dtype), *rows,
+                  *common)
         return (out, lse) if return_lse else out
 
     def forward(self, q: torch.Tensor, paged_kv_cache: torch.Tensor,
@@ -926,11 +947,12 @@ class BatchPrefillWithPagedKVCacheWrapper(_WrapperBase):
             raise ValueError("out must be a contiguous [nnz, num_qo_heads, head_dim] tensor")
         if return_lse and lse is None:
             lse = torch.empty((n, self._hq), dtype=torch.float32, device=q.device)
-        call("pagedattn_prefill_run", self._plan.handle, ptr(q), q.stride(0), q.stride(1),
-             dtype_code(q.dtype), ptr(self._qo_indptr), ptr(paged_kv_cache),
-             dtype_code(paged_kv_cache.dtype), ptr(scales), num_pages, ptr(self._indices),
-             self._indices.numel(), ptr(self._indptr), ptr(self._last), ptr(out), ptr(lse),
-             int(is_causal), float(scale), _stream(q.device))
+        _run_plan("pagedattn_prefill_run", "pagedattn_prefill_run_scratch",
+                  _scratch(self._plan, q.device), q.device, self._plan.handle, ptr(q), q.stride(0),
+                  q.stride(1), dtype_code(q.dtype), ptr(self._qo_indptr), ptr(paged_kv_cache),
+                  dtype_code(paged_kv_cache.dtype), ptr(scales), num_pages, ptr(self._indices),
+                  self._indices.numel(), ptr(self._indptr), ptr(self._last), ptr(out), ptr(lse),
+                  int(is_causal), float(scale))
         return (out, lse) if return_lse else out
 
     def forward(self, q: torch.Tensor, paged_kv_cache: torch.Tensor, causal: bool = False,

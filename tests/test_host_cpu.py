@@ -104,6 +104,27 @@ def test_empty_device_prefill_plan_runs(ws_bytes):
         lib.pagedattn_plan_destroy(plan)
 
 
+def test_scratch_of_device_prefill_plans():
+    # the workspace's size bounds the scratch a plan asks of its runs
+    lib = _lib.lib()
+    plan = lib.pagedattn_plan_create()
+    cus = max(lib.pagedattn_device_cu_count(), 0) or 256
+    try:
+        assert lib.pagedattn_plan_scratch_bytes(plan) == 0
+        for d in (64, 128):
+            need = cus * 256 * (d + 1) * 4
+            for ws_bytes, want in ((need + 255, 0), (need + 256, need), (1 << 16, 0)):
+                assert lib.pagedattn_prefill_plan_device(plan, 3, 32, 8, d, 16, 512,
+                                                         ctypes.c_void_p(1 << 20), ws_bytes) == 0
+                assert lib.pagedattn_plan_scratch_bytes(plan) == want
+        # a plan object's next plan starts over
+        assert lib.pagedattn_decode_plan_device(plan, 4, 32, 8, 64, 16,
+                                                ctypes.c_void_p(1 << 20), 1 << 27) == 0
+        assert lib.pagedattn_plan_scratch_bytes(plan) == 0
+    finally:
+        lib.pagedattn_plan_destroy(plan)
+
+
 def test_wrappers_require_device_tensors():
     ws = torch.zeros(1024, dtype=torch.uint8)
     with pytest.raises(ValueError, match="device"):
