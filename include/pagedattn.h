@@ -266,9 +266,11 @@ void pagedattn_plan_destroy(pagedattn_plan* plan);
  * memory: device scratch of at least this many bytes (256-byte aligned, any
  * contents, used in stream order until the run has ended; at most the
  * workspace's size, which bounds it at plan time).  Runs without scratch, and
- * the calls without the argument, take the whole form.  0: the plan has one
- * form, and scratch is ignored.  The two forms round differently. */
-size_t pagedattn_plan_scratch_bytes(const pagedattn_plan* plan);
+ * the calls without the argument, take the whole form.  0: this run has one
+ * form, and needs no scratch.  The two forms round differently.  q_rows is the
+ * run's rows of q (device prefill plans: too many rows to be cut give 0, so a
+ * full step has no merge launch). */
+size_t pagedattn_plan_scratch_bytes(const pagedattn_plan* plan, int64_t q_rows);
 
 int pagedattn_decode_plan(pagedattn_plan* plan, const int32_t* kv_indptr_host,
                           const int32_t* kv_last_page_len_host,
@@ -457,8 +459,9 @@ int pagedattn_prefill_plan(pagedattn_plan* plan, const int32_t* qo_indptr_host,
  * the plan's fixed capacity of ceil(max_qo_tokens / q_tile) + batch_size tiles
  * (a run with scratch: at least one workgroup per CU, then the merge launch);
  * entries past the run's tiles return at once.  The outputs equal those of a
- * host plan with a workspace of the same size, run like this one with or
- * without scratch, bit for bit.  Tiles beyond the capacity (a run with more than
+ * host plan with a workspace of the same size bit for bit, where the run brings
+ * scratch as the host plan's does (pagedattn_plan_scratch_bytes with the rows of
+ * the step: q with more rows than the step has tokens may say 0).  Tiles beyond the capacity (a run with more than
  * max_qo_tokens query tokens) are skipped and counted at byte 12 of the
  * workspace.  batch_size <= 4096. */
 int pagedattn_prefill_plan_device(pagedattn_plan* plan, int32_t batch_size,

@@ -193,7 +193,7 @@ struct Scratch {
   void* ptr = nullptr;
   size_t bytes = 0;
   void get(const pagedattn_plan* plan, const at::Tensor& q) {
-    bytes = g_entry.scratch_bytes(plan);
+    bytes = g_entry.scratch_bytes(plan, q.size(0));
     if (!bytes) return;
     try {
       t = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte).requires_grad(false));

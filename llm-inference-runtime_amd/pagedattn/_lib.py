@@ -92,7 +92,7 @@ _SIGNATURES = {
         [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,
          _c_p, _c_f, _c_f, _c_p, _c_int, _c_p, _c_int, _c_p, _c_int, _c_p, _c_p, _c_p, _c_p,
          _c_f, _c_p]),
-    "pagedattn_plan_scratch_bytes": (_c_sz, [_c_p]),
+    "pagedattn_plan_scratch_bytes": (_c_sz, [_c_p, _c_i64]),
     "pagedattn_decode_run_scratch": (
         _c_int,
         [_c_p, _c_p, _c_i64, _c_i64, _c_int, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,

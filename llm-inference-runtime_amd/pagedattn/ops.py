@@ -114,16 +114,16 @@ def _native(fn: str, entry: str, *args):
     return r
 
 
-def _scratch(plan: "_Plan", device: torch.device) -> torch.Tensor | None:
+def _scratch(plan: "_Plan", q: torch.Tensor) -> torch.Tensor | None:
     """One run's scratch for the partials of a plan that cuts KV ranges, from
     torch's caching allocator (per run and stream: runs of one plan may
     overlap); None where the plan needs none, or where there is no memory for it
     and the run takes the plan's whole form."""
-    n = _lib.lib().pagedattn_plan_scratch_bytes(plan.handle)
+    n = _lib.lib().pagedattn_plan_scratch_bytes(plan.handle, q.shape[0])
     if n == 0:
         return None
     try:
-        return torch.empty(n, dtype=torch.uint8, device=device)
+        return torch.empty(n, dtype=torch.uint8, device=q.device)
     except torch.OutOfMemoryError:
         return None
 
@@ -792,7 +792,7 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
             rows = (ptr(append_key), ptr(append_value), append_key.stride(0),
                     append_key.stride(1), append_value.stride(0), append_value.stride(1),
                     *rotate)
-        _run_plan(entry, "pagedattn_decode_run_scratch", _scratch(self._plan, q.device), q.device,
+        _run_plan(entry, "pagedattn_decode_run_scratch", _scratch(self._plan, q), q.device,
                   self._plan.handle, ptr(q), q.stride(0), q.stride(1), dtype_code(q.dtype), *rows,
                   *common)
         return (out, lse) if return_lse else out
@@ -819,7 +819,8 @@ class BatchPrefillWithPagedKVCacheWrapper(_WrapperBase):
     was planned with, in their current contents, on the device, for up to n
     query tokens per run, so a chunked-prefill step can be captured in a HIP
     graph and replayed while the metadata changes in place.  The outputs are
-    those of a host plan, bit for bit."""
+    those of a host plan, bit for bit, where q holds just the step's tokens
+    (rows past them may keep a step's KV ranges whole that a host plan cuts)."""
 
     def plan(self, qo_indptr: torch.Tensor, paged_kv_indptr: torch.Tensor,
              paged_kv_indices: torch.Tensor, paged_kv_last_page_len: torch.Tensor,
@@ -948,7 +949,7 @@ class BatchPrefillWithPagedKVCacheWrapper(_WrapperBase):
         if return_lse and lse is None:
             lse = torch.empty((n, self._hq), dtype=torch.float32, device=q.device)
         _run_plan("pagedattn_prefill_run", "pagedattn_prefill_run_scratch",
-                  _scratch(self._plan, q.device), q.device, self._plan.handle, ptr(q), q.stride(0),
+                  _scratch(self._plan, q), q.device, self._plan.handle, ptr(q), q.stride(0),
                   q.stride(1), dtype_code(q.dtype), ptr(self._qo_indptr), ptr(paged_kv_cache),
                   dtype_code(paged_kv_cache.dtype), ptr(scales), num_pages, ptr(self._indices),
                   self._indices.numel(), ptr(self._indptr), ptr(self._last), ptr(out), ptr(lse),

@@ -46,7 +46,7 @@ def _wrapper(gpu, kind, ws=None):
 
 
 def _scratch_bytes(w):
-    return _lib.lib().pagedattn_plan_scratch_bytes(w._plan.handle)
+    return _lib.lib().pagedattn_plan_scratch_bytes(w._plan.handle, 1)
 
 
 @pytest.mark.parametrize("kind", ["decode", "host", "device"])

@@ -265,6 +265,31 @@ def test_chunked_prefill_step_graph_replay(gpu, table):
         assert lse_err(eager.lse[rows], ref_l) <= TOL_LSE, b
 
 
+def test_prefill_device_plan_cuts_only_runs_of_few_rows(gpu, monkeypatch):
+    """One device plan with room for a full step: a run of a few rows is cut and
+    a run of more tiles than slots (CUs / KV heads) has one form, both with the
+    host plan's bits."""
+    monkeypatch.delenv("PAGEDATTN_PREFILL_SPLIT", raising=False)
+    lib = pagedattn.lib()
+    hq, hkv, d = 32, 8, 128
+    most = lib.pagedattn_device_cu_count() // hkv * 64
+    for step, cut in (([(5000, 64)], True), ([(2000, most // 2), (900, most // 2 + 1)], False)):
+        rng = np.random.default_rng(1)
+        tables, num_pages = random_tables(rng, [c + n for c, n in step])
+        meta = prefill_metadata(tables, [c for c, _ in step], [n for _, n in step])
+        pool = torch.randn((num_pages, 2, hkv, 16, d), device=gpu).to(torch.bfloat16)
+        q = torch.randn((meta.nnz, hq, d), device=gpu).to(torch.bfloat16)
+        args = [i32(a, gpu) for a in (meta.qo_indptr, meta.kv_indptr, meta.kv_indices,
+                                      meta.kv_last_page_len)]
+        res = []
+        for kw in (dict(device_plan=True, max_qo_tokens=4 * most), {}):
+            w = pagedattn.BatchPrefillWithPagedKVCacheWrapper(workspace(gpu), "HND")
+            w.plan(*args, hq, hkv, d, 16, causal=True, q_data_type=q.dtype, **kw)
+            assert (lib.pagedattn_plan_scratch_bytes(w._plan.handle, meta.nnz) > 0) == cut
+            res.append(w.run(q, pool, return_lse=True))
+        assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1], res[1][1])
+
+
 @pytest.mark.parametrize("d,hq,hkv", [(128, 32, 8), (64, 32, 4), (128, 12, 3)])
 def test_prefill_device_plan_cuts_kv_like_the_host_plan(gpu, d, hq, hkv):
     """Steps whose KV ranges are cut, steps kept whole and an empty one, one

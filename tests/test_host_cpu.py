@@ -105,22 +105,28 @@ def test_empty_device_prefill_plan_runs(ws_bytes):
 
 
 def test_scratch_of_device_prefill_plans():
-    # the workspace's size bounds the scratch a plan asks of its runs
+    # the workspace's size bounds the scratch a plan asks of its runs, and only
+    # runs of at most one tile per slot (CUs / KV heads) can be cut
     lib = _lib.lib()
     plan = lib.pagedattn_plan_create()
     cus = max(lib.pagedattn_device_cu_count(), 0) or 256
+    ws = ctypes.c_void_p(1 << 20)
+
+    def scratch(rows):
+        return lib.pagedattn_plan_scratch_bytes(plan, rows)
+
     try:
-        assert lib.pagedattn_plan_scratch_bytes(plan) == 0
-        for d in (64, 128):
+        assert scratch(1) == 0
+        for hkv, d in ((4, 64), (8, 128)):
+            most = cus // hkv * (256 // (32 // hkv))
             need = cus * 256 * (d + 1) * 4
             for ws_bytes, want in ((need + 255, 0), (need + 256, need), (1 << 16, 0)):
-                assert lib.pagedattn_prefill_plan_device(plan, 3, 32, 8, d, 16, 512,
-                                                         ctypes.c_void_p(1 << 20), ws_bytes) == 0
-                assert lib.pagedattn_plan_scratch_bytes(plan) == want
+                assert lib.pagedattn_prefill_plan_device(plan, 3, 32, hkv, d, 16, 8 * most, ws,
+                                                         ws_bytes) == 0
+                assert [scratch(r) for r in (0, 1, most, most + 1, 8 * most)] == [want] * 3 + [0, 0]
         # a plan object's next plan starts over
-        assert lib.pagedattn_decode_plan_device(plan, 4, 32, 8, 64, 16,
-                                                ctypes.c_void_p(1 << 20), 1 << 27) == 0
-        assert lib.pagedattn_plan_scratch_bytes(plan) == 0
+        assert lib.pagedattn_decode_plan_device(plan, 4, 32, 8, 64, 16, ws, 1 << 27) == 0
+        assert scratch(1) == 0
     finally:
         lib.pagedattn_plan_destroy(plan)
 
