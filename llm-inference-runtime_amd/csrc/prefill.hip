@@ -726,7 +726,11 @@ struct PrefillMergeArgs {
 };
 
 constexpr int kPrefillMergeWaves = 4;
-constexpr int kPrefillMergeGrid = 2048;  // workgroups: one resident set of waves
+// Workgroups at most: one resident set on 256 CUs (110 VGPRs: 4 waves a SIMD, 4
+// workgroups a CU).  A 512-token chunk over 6100 (32/8 heads, D = 128) takes
+// 74.9 / 69.2 / 66.4 / 67.8 us with 256 / 512 / 1024 / 2048, a device-planned
+// step with nothing to merge 10.4 / 10.4 / 10.5 / 10.7 us.
+constexpr int kPrefillMergeGrid = 1024;
 
 template <bool BF16, int D>
 __global__ void __launch_bounds__(kWave * kPrefillMergeWaves)
