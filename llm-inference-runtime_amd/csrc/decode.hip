@@ -1319,20 +1319,34 @@ __global__ void __launch_bounds__(256, 1) decode_shared_kernel(DecodeParams p) {
 // Combine the base-2 partials of n pieces, slot_of(s) giving piece s's
 // (slot * g + head) index: M = max lse, den = sum 2^(lse - M), num = sum
 // 2^(lse - M) o, out = num / den.  Pieces s, s + 8, s + 16, ... form class
-// s mod 8; a wave sums a class, kMergeBatch loads at a time, and the classes
-// are added in order, so the bits depend on the piece count alone and not on
-// the workgroup's waves (any number from D / 64 to 8).  A piece with a NaN lse
-// makes the row NaN with lse = -inf, as an uncut item writes it; with no score
-// at all den and num are 0.
+// s mod 8; a class is summed kMergeBatch pieces at a time, and the classes are
+// added in order, so the bits depend on the piece count alone and not on the
+// workgroup: eight waves, one per class (EIGHT), or D threads, one per d.  A
+// piece with a NaN lse makes the row NaN with lse = -inf, as an uncut item
+// writes it; with no score at all den and num are 0.
 //
 // Bound by the latency of dependent loads, not by bytes (a partial row is
-// 256-512 B): one thread per d walking the pieces four at a time took 24
-// round trips for the 94 pieces of one long sequence; eight waves of eight
-// loads take 64 pieces per round trip.  Up to 8 pieces are one round trip
-// of D threads, with no LDS and no barrier: a batch of mixed lengths has
-// about a thousand such rows, and eight waves for each cost 1.5 us more.
+// 256-512 B).  D threads take 16 pieces per round trip, up to 8 pieces with no
+// loop, eight waves 64; but eight waves for each of the 512 / 1024 / 2048 rows of
+// an even batch cost 0.7 / 1.8 / 4 us more than D threads (18.6 / 18.6 / 20.0 us
+// against 18.1 / 17.0 / 16.3 us, 32 heads, D = 128, 500 to 128 tokens).
 constexpr int kMergeClasses = 8;
 constexpr int kMergeBatch = 8;
+constexpr int kMergeLoads = 16;
+static_assert(kMergeClasses * kMergeBatch == kWave, "one piece's lse per lane");
+// So eight waves merge a launch of at most 16 rows per piece of its longest row:
+// one sequence of 32000 tokens among 15 of 1000 (512 rows, 87 pieces) runs 42.3 us
+// with eight waves and 47.4 us with D threads, 24 equal ones of 2730 (768 rows,
+// 10 pieces) 53.0 and 51.6 us.  Device partitions do not know their pieces: 256
+// rows, one per CU (8 sequences of 4000 tokens 15.2 against 15.9 us, of 500 12.4
+// against 12.2 us).
+constexpr int kMergeRowsPerPiece = 16;
+constexpr int kMergeDeviceRows = 256;
+
+__device__ __forceinline__ float merge_lane(float v, int i) {
+  return __builtin_bit_cast(float,
+                            __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i));
+}
 
 template <bool BF16>
 __device__ __forceinline__ void merge_write(float M, float num, float den, int dd, uint16_t* orow,
@@ -1342,7 +1356,7 @@ __device__ __forceinline__ void merge_write(float M, float num, float den, int d
     *lse = den > 0.f ? (M + log2f(den)) * 0.69314718055994531f : -INFINITY;
 }
 
-template <bool BF16, int D, typename SlotOf>
+template <bool BF16, int D, bool EIGHT, typename SlotOf>
 __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float* __restrict__ pl,
                                              const float* __restrict__ po, uint16_t* orow,
                                              float* lse) {
@@ -1372,10 +1386,61 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
     merge_write<BF16>(M, num, den, dd, orow, lse);
     return;
   }
-  __shared__ float s_m[kMergeClasses], s_den[kMergeClasses], s_num[kMergeClasses][D];
-  const int wave = uniform(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  for (int cls = wave; cls < kMergeClasses; cls += blockDim.x >> 6) {
+  if constexpr (!EIGHT) {
+    // lane i holds piece base + i's lse and weight, and class i mod 8's M and den
+    float Mc = -INFINITY, den = 0.f, num[kMergeClasses];
+#pragma unroll
+    for (int c = 0; c < kMergeClasses; ++c) num[c] = 0.f;
+    for (int base = 0; base < n; base += kWave) {
+      const int nb = min(n - base, kWave);
+      float lv = -INFINITY, ov[kMergeLoads];
+      auto load = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < kMergeLoads; ++i) {
+          ov[i] = 0.f;
+          if (i0 + i < nb) ov[i] = po[slot_of(base + i0 + i) * D + dd];
+        }
+      };
+      if (lane < nb) lv = pl[slot_of(base + lane)];
+      load(0);
+      float Mb = fmaxf(Mc, lv);
+#pragma unroll
+      for (int off = kMergeClasses; off < kWave; off <<= 1) Mb = fmaxf(Mb, __shfl_xor(Mb, off));
+      const float r = Mc == -INFINITY ? 0.f : exp2f(Mc - Mb);
+      const float wt = lv == -INFINITY ? 0.f : exp2f(lv - Mb);
+      den *= r;
+#pragma unroll
+      for (int k = 0; k < kMergeBatch; ++k)
+        den += __shfl(wt, kMergeClasses * k + (lane & (kMergeClasses - 1)));
+#pragma unroll
+      for (int c = 0; c < kMergeClasses; ++c) num[c] *= merge_lane(r, c);
+      for (int i0 = 0;;) {
+#pragma unroll
+        for (int i = 0; i < kMergeLoads; ++i)
+          num[i % kMergeClasses] = fmaf(merge_lane(wt, i0 + i), ov[i], num[i % kMergeClasses]);
+        i0 += kMergeLoads;
+        if (i0 >= nb) break;
+        load(i0);
+      }
+      Mc = Mb;
+    }
+    float M = Mc;
+#pragma unroll
+    for (int off = 1; off < kMergeClasses; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
+    const float wc = Mc == -INFINITY ? 0.f : exp2f(Mc - M);
+    float dsum = 0.f, nsum = 0.f;
+#pragma unroll
+    for (int c = 0; c < kMergeClasses; ++c) {
+      dsum = fmaf(merge_lane(wc, c), merge_lane(den, c), dsum);
+      nsum = fmaf(merge_lane(wc, c), num[c], nsum);
+    }
+    merge_write<BF16>(M, nsum, dsum, dd, orow, lse);
+    return;
+  }
+  __shared__ float s_m[kMergeClasses], s_den[kMergeClasses], s_num[kMergeClasses][D];
+  const int cls = uniform(threadIdx.x >> 6);
+  {
     float M = -INFINITY, den = 0.f, num[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) num[e] = 0.f;
@@ -1436,8 +1501,8 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
 // lse = M + log2(sum_c 2^(lse_c - M)) (base-2 partials, natural-log output).
 // A separate launch: the kernel boundary orders the partial writes before
 // these reads across the XCDs' L2 caches without per-item cache flushes.
-template <bool BF16, int D>
-__global__ void __launch_bounds__(kWave * kMergeClasses)
+template <bool BF16, int D, bool EIGHT>
+__global__ void __launch_bounds__(EIGHT ? kWave * kMergeClasses : D)
     decode_merge_kernel(const MergeItem* __restrict__ merges,
                         const float* __restrict__ po,
                         const float* __restrict__ pl, uint16_t* __restrict__ out,
@@ -1445,7 +1510,7 @@ __global__ void __launch_bounds__(kWave * kMergeClasses)
   const MergeItem mi = merges[blockIdx.x];
   const int hn = blockIdx.y;  // query head within the group
   const int64_t row = (int64_t)mi.b * hq + mi.h * g + hn;
-  merge_pieces<BF16, D>(
+  merge_pieces<BF16, D, EIGHT>(
       mi.nslots, [&](int s) { return (int64_t)(mi.slot0 + s * mi.stride) * g + hn; }, pl, po,
       out + row * D, lse ? lse + row : nullptr);
 }
@@ -1466,8 +1531,8 @@ struct MergeImplicitArgs {
   int32_t batch, hq, hkv, g, hg_shift, n_groups, item_cost;
 };
 
-template <bool BF16, int D>
-__global__ void __launch_bounds__(kWave * kMergeClasses)
+template <bool BF16, int D, bool EIGHT>
+__global__ void __launch_bounds__(EIGHT ? kWave * kMergeClasses : D)
     decode_merge_implicit_kernel(MergeImplicitArgs a) {
   const int b = blockIdx.x / a.hkv;
   const int h = blockIdx.x % a.hkv;
@@ -1495,7 +1560,7 @@ __global__ void __launch_bounds__(kWave * kMergeClasses)
     const int j = (w == first && p0 != w * sp.share) ? 1 : 0;
     return ((2 * w + j) << a.hg_shift) + wi;
   };
-  merge_pieces<BF16, D>(
+  merge_pieces<BF16, D, EIGHT>(
       (int)(last - first + 1), [&](int s) { return slot_of(first + s) * a.g + hn; }, a.pl, a.po,
       orow, a.lse ? a.lse + (int64_t)b * a.hq + head : nullptr);
 }
@@ -1551,6 +1616,17 @@ static DecodeFn pick_decode(int d, bool bf16, bool fp8, bool append, bool rope, 
                     : decode_fn_d<64, false>(bf16, fp8, append, rope);
   return implicit ? decode_fn_d<128, true>(bf16, fp8, append, rope)
                   : decode_fn_d<128, false>(bf16, fp8, append, rope);
+}
+
+template <bool BF16, int D>
+static auto pick_merge(bool eight) {
+  return eight ? decode_merge_kernel<BF16, D, true> : decode_merge_kernel<BF16, D, false>;
+}
+
+template <bool BF16, int D>
+static auto pick_merge_implicit(bool eight) {
+  return eight ? decode_merge_implicit_kernel<BF16, D, true>
+               : decode_merge_implicit_kernel<BF16, D, false>;
 }
 
 }  // namespace pa
@@ -1685,23 +1761,23 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
                         plan->batch_size, plan->hq, plan->hkv, p.g,
                         plan->hg_shift, plan->n_items, plan->item_cost};
     const dim3 grid((unsigned)((int64_t)plan->batch_size * plan->hkv), p.g);
-    auto* mfn = plan->d == 64 ? (bf16 ? decode_merge_implicit_kernel<true, 64>
-                                      : decode_merge_implicit_kernel<false, 64>)
-                              : (bf16 ? decode_merge_implicit_kernel<true, 128>
-                                      : decode_merge_implicit_kernel<false, 128>);
-    // piece counts are only known on the device: eight waves a row while the
-    // rows are too few to fill the GPU by themselves
-    const int64_t rows = (int64_t)plan->batch_size * plan->hq;
-    hipLaunchKernelGGL(mfn, grid, dim3(rows <= 1024 ? kWave * kMergeClasses : plan->d), 0, s, m);
+    const bool eight = (int64_t)plan->batch_size * plan->hq <= kMergeDeviceRows;
+    auto* mfn = plan->d == 64 ? (bf16 ? pick_merge_implicit<true, 64>(eight)
+                                      : pick_merge_implicit<false, 64>(eight))
+                              : (bf16 ? pick_merge_implicit<true, 128>(eight)
+                                      : pick_merge_implicit<false, 128>(eight));
+    hipLaunchKernelGGL(mfn, grid, dim3(eight ? kWave * kMergeClasses : plan->d), 0, s, m);
     return check_launch("decode_run(merge)");
   }
   if (plan->n_merge == 0) return rc;
   const dim3 grid(plan->n_merge, p.g);
+  const bool eight =
+      plan->max_pieces > kMergeClasses &&
+      (int64_t)plan->n_merge * p.g <= (int64_t)kMergeRowsPerPiece * plan->max_pieces;
   auto* mfn = plan->d == 64
-                  ? (bf16 ? decode_merge_kernel<true, 64> : decode_merge_kernel<false, 64>)
-                  : (bf16 ? decode_merge_kernel<true, 128> : decode_merge_kernel<false, 128>);
-  hipLaunchKernelGGL(mfn, grid,
-                     dim3(plan->max_pieces > kMergeClasses ? kWave * kMergeClasses : plan->d), 0, s,
+                  ? (bf16 ? pick_merge<true, 64>(eight) : pick_merge<false, 64>(eight))
+                  : (bf16 ? pick_merge<true, 128>(eight) : pick_merge<false, 128>(eight));
+  hipLaunchKernelGGL(mfn, grid, dim3(eight ? kWave * kMergeClasses : plan->d), 0, s,
                      static_cast<const MergeItem*>(plan->merge_dev), p.partial_o, p.partial_lse,
                      p.out, lse, plan->hq, p.g);
   return check_launch("decode_run(merge)");

@@ -69,10 +69,12 @@ def test_decode_balanced_item_cost(gpu, monkeypatch, cost):
 
 
 @pytest.mark.parametrize("d", [64, 128])
-@pytest.mark.parametrize("pieces", [[8, 3, 1], [9, 8, 2], [16, 17], [63, 65, 1]])
+@pytest.mark.parametrize("pieces", [[8, 3, 1], [9, 8, 2], [16, 17], [63, 65, 1],
+                                    [17, 16] + [9] * 19, [66, 65] + [2] * 70])
 def test_decode_merge_piece_counts(gpu, d, pieces):
     # fixed chunks of 128 tokens: up to 8 pieces a row (one round trip of the
-    # merge), one past it, and around its 64 pieces per round trip
+    # merge), one past it, and around its 64 pieces per round trip; in the last
+    # two, rows enough for D threads a row (16 and 64 pieces per round trip)
     lens = [128 * n - (5 if n > 1 else 100) for n in pieces]
     meta, pool, q = decode_case(gpu, lens, 16, 2, d, seed=sum(pieces))
     ref_o, ref_l = oracle_decode(meta, pool, q)
@@ -84,7 +86,7 @@ def test_decode_merge_piece_counts(gpu, d, pieces):
 @pytest.mark.parametrize("lens,hq", [([9001], 16), ([9001] + [20] * 69, 16)])
 def test_decode_device_plan_one_long_sequence(gpu, lens, hq):
     # the device partition's merge over many pieces, with eight waves a row
-    # (few rows) and with D threads a row (more than 1024 rows)
+    # (few rows) and with D threads a row (more than 256 rows)
     meta, pool, q = decode_case(gpu, lens, hq, 2, 128, seed=len(lens))
     ref_o, ref_l = oracle_decode(meta, pool, q)
     w = pagedattn.BatchDecodeWithPagedKVCacheWrapper(workspace(gpu), "HND")
