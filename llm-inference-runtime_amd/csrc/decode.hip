@@ -1338,7 +1338,7 @@ static_assert(kMergeClasses * kMergeBatch == kWave, "one piece's lse per lane");
 // one sequence of 32000 tokens among 15 of 1000 (512 rows, 87 pieces) runs 42.3 us
 // with eight waves and 47.4 us with D threads, 24 equal ones of 2730 (768 rows,
 // 10 pieces) 53.0 and 51.6 us.  Device partitions do not know their pieces: 256
-// rows, one per CU (8 sequences of 4000 tokens 15.2 against 15.9 us, of 500 12.4
+// rows, one per CU (8 sequences of 4000 tokens 14.8 against 15.9 us, of 500 12.5
 // against 12.2 us).
 constexpr int kMergeRowsPerPiece = 16;
 constexpr int kMergeDeviceRows = 256;
@@ -1445,33 +1445,35 @@ __device__ __forceinline__ void merge_pieces(int n, SlotOf slot_of, const float*
 #pragma unroll
     for (int e = 0; e < V; ++e) num[e] = 0.f;
     for (int s0 = cls; s0 < n; s0 += kMergeClasses * kMergeBatch) {
-      float lv[kMergeBatch], ov[kMergeBatch][V];
+      // lane i: the lse and weight of the batch's piece i mod 8 (one load for all
+      // of them: as scalar loads each was waited for, 0.6 us a launch)
+      float lv = -INFINITY, ov[kMergeBatch][V];
+      const int s_lane = s0 + kMergeClasses * (lane & (kMergeBatch - 1));
+      if (s_lane < n) lv = pl[slot_of(s_lane)];
 #pragma unroll
       for (int k = 0; k < kMergeBatch; ++k) {
         const int s = s0 + kMergeClasses * k;
-        lv[k] = -INFINITY;
 #pragma unroll
         for (int e = 0; e < V; ++e) ov[k][e] = 0.f;
         if (s < n) {
           const int64_t sh = slot_of(s);
-          lv[k] = pl[sh];
 #pragma unroll
           for (int e = 0; e < V; ++e) ov[k][e] = po[sh * D + V * lane + e];
         }
       }
-      float Mb = M;
+      float Mb = fmaxf(M, lv);
 #pragma unroll
-      for (int k = 0; k < kMergeBatch; ++k) Mb = fmaxf(Mb, lv[k]);
+      for (int off = 1; off < kMergeBatch; off <<= 1) Mb = fmaxf(Mb, __shfl_xor(Mb, off));
       const float r = M == -INFINITY ? 0.f : exp2f(M - Mb);
+      const float wt = lv == -INFINITY ? 0.f : exp2f(lv - Mb);
       den *= r;
 #pragma unroll
       for (int e = 0; e < V; ++e) num[e] *= r;
 #pragma unroll
       for (int k = 0; k < kMergeBatch; ++k) {
-        const float wt = lv[k] == -INFINITY ? 0.f : exp2f(lv[k] - Mb);
-        den += wt;
+        den += merge_lane(wt, k);
 #pragma unroll
-        for (int e = 0; e < V; ++e) num[e] = fmaf(wt, ov[k][e], num[e]);
+        for (int e = 0; e < V; ++e) num[e] = fmaf(merge_lane(wt, k), ov[k][e], num[e]);
       }
       M = Mb;
     }
