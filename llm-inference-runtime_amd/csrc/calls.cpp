@@ -17,6 +17,8 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/Allocator.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/util/Exception.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -189,15 +191,16 @@ struct Outputs {
 // one plan may overlap; freed when the call returns, it is reused in stream
 // order.  Without memory for it the run takes the plan's whole form.
 struct Scratch {
-  at::Tensor t;
+  c10::DataPtr mem;
   void* ptr = nullptr;
   size_t bytes = 0;
   void get(const pagedattn_plan* plan, const at::Tensor& q) {
     bytes = g_entry.scratch_bytes(plan, q.size(0));
     if (!bytes) return;
     try {
-      t = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte).requires_grad(false));
-      ptr = t.data_ptr();
+      const c10::DeviceGuard guard(q.device());
+      mem = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(bytes);
+      ptr = mem.get();
     } catch (const c10::OutOfMemoryError&) {
       bytes = 0;
     }
