@@ -146,15 +146,18 @@ struct Outputs {
       out = at::empty({n, hq, d}, q.options().requires_grad(false));
     } else {
       const at::Tensor* t = plain(o);
-      if (!t || !t->is_cuda() || !t->is_contiguous() || t->dim() != 3 || t->size(0) != n ||
-          t->size(1) != hq || t->size(2) != d)
+      if (!t || t->device() != q.device() || t->scalar_type() != q.scalar_type() ||
+          !t->is_contiguous() || t->dim() != 3 || t->size(0) != n || t->size(1) != hq ||
+          t->size(2) != d)
         return false;
       out = *t;
       out_o = o;
     }
     if (l != Py_None) {
       const at::Tensor* t = plain(l);
-      if (!t) return false;
+      if (!t || t->device() != q.device() || t->scalar_type() != at::kFloat ||
+          !t->is_contiguous() || t->numel() < n * hq)
+        return false;
       lse = *t;
       lse_o = l;
       lse_ptr = lse.data_ptr();

@@ -149,6 +149,19 @@ def _check_rows(x: torch.Tensor, name: str, heads: int | None, d: int | None):
         raise ValueError(f"{name}: the head_dim axis must be contiguous")
 
 
+def _check_outputs(out: torch.Tensor | None, lse: torch.Tensor | None, q: torch.Tensor,
+                   shape: tuple[int, int, int], names: str) -> None:
+    """The caller's out and lse, written through their raw pointers."""
+    if out is not None and (not out.is_contiguous() or tuple(out.shape) != shape
+                            or out.dtype != q.dtype or out.device != q.device):
+        raise ValueError(f"out must be a contiguous [{names}, num_qo_heads, head_dim] tensor in "
+                         "q's dtype and on its device")
+    if lse is not None and (lse.dtype != torch.float32 or not lse.is_contiguous()
+                            or lse.device != q.device or lse.numel() < shape[0] * shape[1]):
+        raise ValueError(f"lse must be a contiguous float32 [{names}, num_qo_heads] tensor on "
+                         "q's device")
+
+
 # -----------------------------------------------------------------------------
 def get_batch_indices_positions(append_indptr: torch.Tensor, seq_lens: torch.Tensor,
                                 nnz: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -759,10 +772,9 @@ class BatchDecodeWithPagedKVCacheWrapper(_WrapperBase):
         if q.dtype not in (torch.float16, torch.bfloat16):
             raise NotImplementedError(f"q dtype {q.dtype}")
         scales = _check_scales(kv_scales, paged_kv_cache)
+        _check_outputs(out, lse, q, (self._bsz, self._hq, self._d), "batch")
         if out is None:
             out = torch.empty((self._bsz, self._hq, self._d), dtype=q.dtype, device=q.device)
-        elif not out.is_contiguous() or tuple(out.shape) != (self._bsz, self._hq, self._d):
-            raise ValueError("out must be a contiguous [batch, num_qo_heads, head_dim] tensor")
         if return_lse and lse is None:
             lse = torch.empty((self._bsz, self._hq), dtype=torch.float32, device=q.device)
         common = (ptr(paged_kv_cache), dtype_code(paged_kv_cache.dtype), ptr(scales),
@@ -942,10 +954,9 @@ class BatchPrefillWithPagedKVCacheWrapper(_WrapperBase):
             raise NotImplementedError(f"q dtype {q.dtype}")
         scales = _check_scales(kv_scales, paged_kv_cache)
         n = q.shape[0]
+        _check_outputs(out, lse, q, (n, self._hq, self._d), "nnz")
         if out is None:
             out = torch.empty((n, self._hq, self._d), dtype=q.dtype, device=q.device)
-        elif not out.is_contiguous() or tuple(out.shape) != (n, self._hq, self._d):
-            raise ValueError("out must be a contiguous [nnz, num_qo_heads, head_dim] tensor")
         if return_lse and lse is None:
             lse = torch.empty((n, self._hq), dtype=torch.float32, device=q.device)
         _run_plan("pagedattn_prefill_run", "pagedattn_prefill_run_scratch",

@@ -349,3 +349,37 @@ def test_native_calls_equal_the_general_path(gpu, monkeypatch, dtype, fp8):
         x, y, z = (t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t
                    for t in (x, y, z))
         assert torch.equal(x, y) and torch.equal(x, z)
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_runs_refuse_outputs_they_would_overrun(gpu, monkeypatch, native):
+    # out and lse are written through raw pointers: anything but q's dtype (lse:
+    # float32), enough entries in order and q's device is refused before a launch
+    if not native:
+        monkeypatch.setattr(pagedattn.ops, "_native", lambda *a: NotImplemented)
+    hq, hkv, d = 8, 2, 64
+    meta = prefill_metadata([[0, 1], [2, 3]], [10, 20], [2, 3])
+    pool = torch.zeros((4, 2, hkv, 16, d), dtype=torch.bfloat16, device=gpu)
+    args = [i32(a, gpu) for a in (meta.kv_indptr, meta.kv_indices, meta.kv_last_page_len)]
+    ws = torch.zeros(1 << 20, dtype=torch.uint8, device=gpu)
+    dw = pagedattn.BatchDecodeWithPagedKVCacheWrapper(ws, "HND")
+    dw.plan(*args, hq, hkv, d, 16, q_data_type=torch.bfloat16)
+    pw = pagedattn.BatchPrefillWithPagedKVCacheWrapper(ws.clone(), "HND")
+    pw.plan(i32(meta.qo_indptr, gpu), *args, hq, hkv, d, 16, q_data_type=torch.bfloat16)
+    for w, n in ((dw, 2), (pw, meta.nnz)):
+        q = torch.ones((n, hq, d), dtype=torch.bfloat16, device=gpu)
+        for out in (torch.empty((n, hq, d), dtype=torch.uint8, device=gpu),
+                    torch.empty((n, hq, d), dtype=torch.float16, device=gpu),
+                    torch.empty((n, hq, d), dtype=q.dtype)):
+            with pytest.raises(ValueError, match="out must be"):
+                w.run(q, pool, out=out)
+        for lse in (torch.empty((n, hq)), torch.empty((n, hq), dtype=q.dtype, device=gpu),
+                    torch.empty((n, hq - 1), device=gpu),
+                    torch.empty((n, 2 * hq), device=gpu)[:, ::2]):
+            with pytest.raises(ValueError, match="lse must be"):
+                w.run(q, pool, lse=lse, return_lse=True)
+        # more room than needed, in any shape, is taken as it was
+        big = torch.full((n * hq + 3,), -1.0, device=gpu)
+        out, lse = w.run(q, pool, lse=big, return_lse=True)
+        assert lse is big and torch.equal(big[n * hq:], torch.full((3,), -1.0, device=gpu))
+        assert torch.equal(big[:n * hq].view(n, hq), w.run(q, pool, return_lse=True)[1])
