@@ -289,8 +289,9 @@ def test_rope_append_shapes_equal_separate(gpu, d, hq, hkv, nnz):
 @pytest.mark.parametrize("dtype,fp8", [(torch.bfloat16, False), (torch.float16, False),
                                        (torch.bfloat16, True)])
 def test_native_calls_equal_the_general_path(gpu, monkeypatch, dtype, fp8):
-    # every per-layer call through the extension and, with it switched off,
-    # through the general path: same bits; int64 metadata goes the general way
+    # every per-layer call through the extension, which takes all of them, and,
+    # with it switched off, through the general path: same bits; calls with int64
+    # metadata go the general way
     hq, hkv, d = 8, 2, 64
     g = torch.Generator(device=gpu)
     g.manual_seed(3)
@@ -341,8 +342,22 @@ def test_native_calls_equal_the_general_path(gpu, monkeypatch, dtype, fp8):
         torch.cuda.synchronize()
         return res
 
+    took = []
+    native = pagedattn.ops._native
+
+    def record(fn, *args):
+        r = native(fn, *args)
+        took.append((fn, r is not NotImplemented))
+        return r
+
+    monkeypatch.setattr(pagedattn.ops, "_native", record)
     want = step(lambda t: t)
+    writes = ["append", "rope_append"] + ["append_amax"] * fp8
+    assert took == [(fn, True) for fn in writes + ["prefill_run"] * 2 + ["decode_run"] * 4]
+    took.clear()
     wide = step(lambda t: t.long())
+    assert took == ([(fn, False) for fn in writes] + [("prefill_run", True)] * 2
+                    + [("decode_run", True)] * 3 + [("decode_run", False)])
     monkeypatch.setattr(pagedattn.ops, "_native", lambda *a: NotImplemented)
     general = step(lambda t: t)
     for x, y, z in zip(want, wide, general):
