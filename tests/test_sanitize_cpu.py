@@ -4,8 +4,9 @@ plan(), src/models/llama.py:86-147) built with AddressSanitizer and
 UndefinedBehaviorSanitizer and driven with randomized and malformed metadata
 (tests/sanitize/plan_fuzz.cpp).  Bad metadata must come back as an error
 status, which the Python layer raises (the reference's callers fail the batch,
-process_loop.py:129-132), never as undefined behaviour.  CPU only: without a
-GPU the planners run up to the work-list upload."""
+process_loop.py:129-132), never as undefined behaviour, and the work lists of
+good metadata must agree with it.  CPU only: the work-list upload is a copy into
+host memory."""
 
 import os
 import shutil
