@@ -333,7 +333,7 @@ int pagedattn_decode_plan_device_update(pagedattn_plan* plan, const int32_t* kv_
  * at run time, see pagedattn_decode_plan_device), or 0
  * for a plan that is not a decode plan.  pagedattn_decode_plan with
  * split_pages = 0 takes a shared plan when its busiest CU carries at most
- * PAGEDATTN_DECODE_SHARED_SLACK_KB (environment, default 96, or 120 for fewer
+ * PAGEDATTN_DECODE_SHARED_SLACK_KB (environment, default 96, or 148 for fewer
  * items than CUs) KiB plus PAGEDATTN_DECODE_SHARED_SLACK_PCT (default 4)
  * percent of the mean more K/V than the mean over all CUs.  A plan that is
  * balanced over fewer CUs is a split one for runs with scratch

@@ -61,12 +61,16 @@ static int decode_head_group(int hkv) {
 // CUs.  Measured on the 70B-shaped e4m3 batch (D = 128, busiest CU 3.1 % over
 // the mean): 214 us shared against 225 us split.  Batches of fewer items than
 // CUs leave CUs idle, and the busy ones then stream faster (38 against 26
-// KiB/us each), so their default slack is 120 KiB: equal-length sequences of
-// 128 KiB an item run 8.7-8.9 us either way on 8-64 items (the split's second
-// launch on top where the host launches each step), and 256 KiB an item 10.8
-// us shared against 9.4 us split on 8 items, 14.0 against 12.5 us on 128.
-// One sequence of 9001 tokens over 8 KV heads of D = 128 (4.4 MiB an item on
-// 8 of 256 CUs): 93 us shared, 14 us split.
+// KiB/us each), so their default slack is 148 KiB.  One sequence of 8 KV heads
+// at D = 128, shared against split: 8.4 and 9.8 us at 256 tokens (128 KiB an
+// item), 9.2 and 9.8 us at 300, 9.7 either way at 350 where the host launches
+// each step and waits for the split's second launch; in a HIP graph 8.2 and 8.7
+// us, 8.9 and 8.8 us, 9.8 and 8.8 us.  e4m3 pages count as 16-bit ones: an item
+// of half the bytes takes as many rounds of loads (256 and 350 tokens: 7.0 and
+// 8.1 us shared, 10.5 us split from the host; 7.2 and 8.2 against 7.2 and 7.5 us
+// in a graph).  D = 64 (4 heads) 512 tokens: 7.7 and 9.6 us, in a graph 7.8 and
+// 7.7 us.  One sequence of 9001 tokens over 8 KV heads of D = 128 (4.4 MiB an
+// item on 8 of 256 CUs): 93 us shared, 14 us split.
 static int decode_shared_mode() {
   if (const char* env = std::getenv("PAGEDATTN_DECODE_SHARED")) {
     const int v = std::atoi(env);
@@ -98,7 +102,7 @@ static int64_t decode_shared_slack_bytes(bool idle_cus) {
     const int v = std::atoi(env);
     if (v >= 0) return (int64_t)v << 10;
   }
-  return (int64_t)(idle_cus ? 120 : 96) << 10;
+  return (int64_t)(idle_cus ? 148 : 96) << 10;
 }
 static int decode_shared_slack_pct() {
   if (const char* env = std::getenv("PAGEDATTN_DECODE_SHARED_SLACK_PCT")) {
