@@ -70,7 +70,7 @@ static int decode_head_group(int hkv) {
 // 8.1 us shared, 10.5 us split from the host; 7.2 and 8.2 against 7.2 and 7.5 us
 // in a graph).  D = 64 (4 heads) 512 tokens: 7.7 and 9.6 us, in a graph 7.8 and
 // 7.7 us.  One sequence of 9001 tokens over 8 KV heads of D = 128 (4.4 MiB an
-// item on 8 of 256 CUs): 93 us shared, 14 us split.
+// item on 8 of 256 CUs): 122 us shared, 14 us split.
 static int decode_shared_mode() {
   if (const char* env = std::getenv("PAGEDATTN_DECODE_SHARED")) {
     const int v = std::atoi(env);

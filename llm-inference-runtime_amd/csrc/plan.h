@@ -41,7 +41,7 @@ struct PrefillItem {
 };
 
 // One entry of a split prefill work list: piece k of the n that the KV tiles
-// of query tokens [q_lo, q_hi) of sequence b are cut into (prefill_pieces).
+// of query tokens [q_lo, q_hi) of sequence b are cut into (prefill_split_cost).
 // n = 1: the whole tile, written to the output (`flag` as PrefillItem::slot);
 // n > 1: split partials to slot `slot` of every KV head.
 struct PrefillPiece {
@@ -101,7 +101,13 @@ constexpr int kPrefillDevSortMax = 1024;
 // Measured on steps of 32/8 heads at D = 128, whole and cut: 1 x 8 workgroups
 // of 16 KV tiles 30.7 and 12.5 us; 8 x 8 of 13 28.7 and 24.8 us, of 133 200
 // and 85 us; 16 x 8 of 17 38.5 and 41.7 us (kept whole), of 24 45.7 and 44.7 us,
-// of 141 212 and 157 us.
+// of 141 212 and 157 us.  The same estimate serves the other types, where cutting
+// gains about as much at the same tile counts: e4m3 pools 8 x 8 of 17 40.0 and 29.1
+// us, 16 x 8 of 33 71.2 and 60.5 us; 32/4 heads at D = 64 16 x 4 of 17 24.4 and
+// 19.6 us, 32 x 4 of 33 43.1 and 38.0 us, e4m3 55.2 and 41.6 us; 8/1 heads at D = 128
+// e4m3 32 x 1 of 17 39.4 and 23.7 us.  Of 680 steps of all these heads and types, of
+// 1 to 256 tiles over 64 to 23000 tokens, the rule made one slower by more than 0.3
+// us (73 tiles of 8/1 heads over 95 tokens, fp16: 25.3 and 26.5 us).
 constexpr int kPrefillSplitMaxPieces = 128;
 constexpr int kPrefillSplitMinTiles = 3;
 constexpr int kPrefillKvTile = 64;

@@ -398,3 +398,75 @@ def test_runs_refuse_outputs_they_would_overrun(gpu, monkeypatch, native):
         out, lse = w.run(q, pool, lse=big, return_lse=True)
         assert lse is big and torch.equal(big[n * hq:], torch.full((3,), -1.0, device=gpu))
         assert torch.equal(big[:n * hq].view(n, hq), w.run(q, pool, return_lse=True)[1])
+
+
+def test_native_calls_refuse_what_the_general_path_refuses(gpu, monkeypatch):
+    # the extension repeats the general path's checks: bad device arguments end
+    # in the same errors with it and without it
+    n, hq, hkv, d = 2, 8, 2, 64
+    dev = dict(device=gpu)
+    bf = dict(dtype=torch.bfloat16, **dev)
+    meta = prefill_metadata([[0], [1]], [3, 4], [1, 1])
+    ind, indptr = i32(meta.kv_indices, gpu), i32(meta.kv_indptr, gpu)
+    last, qo = i32(meta.kv_last_page_len, gpu), i32(meta.qo_indptr, gpu)
+    bi, pos = i32(meta.batch_indices, gpu), i32(meta.positions, gpu)
+    pool, q = torch.zeros((2, 2, hkv, 16, d), **bf), torch.ones((n, hq, d), **bf)
+    k = torch.ones((n, hkv, d), **bf)
+    pool8 = torch.zeros(pool.shape, dtype=torch.uint8, **dev).view(torch.float8_e4m3fn)
+    scales = torch.ones((2, 2, hkv), **dev)
+    ws = torch.zeros(1 << 20, dtype=torch.uint8, device=gpu)
+    dw = pagedattn.BatchDecodeWithPagedKVCacheWrapper(ws, "HND")
+    dw.plan(indptr, ind, last, hq, hkv, d, 16, q_data_type=torch.bfloat16)
+    pw = pagedattn.BatchPrefillWithPagedKVCacheWrapper(ws.clone(), "HND")
+    pw.plan(qo, indptr, ind, last, hq, hkv, d, 16, q_data_type=torch.bfloat16)
+    bad_q = [q[:, :4], q[..., :32], q[:1], q.float(), q.to(torch.float16), q[0],
+             torch.ones((n, hq, 2 * d), **bf)[..., ::2]]
+    bad_pool = [pool[:, :1], pool[:, :, :1], pool[..., :32], pool.float(), pool.to(torch.float16),
+                pool[:, :, :, :8], pool[0], torch.zeros((2, 2, hkv, 16, 2 * d), **bf)[..., ::2]]
+    bad_scales = [None, scales[:1], scales.half(), scales.cpu()]
+    bad_rows = [k[:, :1], k[:1], k[..., :32], k.float(), k.to(torch.float16)]
+    meta_args = (bi, pos, pool, ind, indptr, last)
+    rope = dict(rope=(1.0, 1e4))
+    calls = [lambda w=w, x=x: w.run(x, pool) for w in (dw, pw) for x in bad_q]
+    calls += [lambda w=w, x=x: w.run(q, x) for w in (dw, pw) for x in bad_pool]
+    calls += [lambda w=w, x=x: w.run(q, pool8, kv_scales=x) for w in (dw, pw) for x in bad_scales]
+    calls += [lambda x=x, r=r: dw.run(q, pool, append_key=x, append_value=k, **r)
+              for x in bad_rows for r in ({}, rope)]
+    calls += [lambda x=x: dw.run(q, pool, append_key=k, append_value=x) for x in [None] + bad_rows]
+    calls += [lambda: dw.run(q, pool, append_value=k),
+              lambda: dw.run(q, pool, append_key=k, append_value=k, positions=pos),
+              lambda: dw.run(q, pool, append_key=k, append_value=k, positions=pos[:1], **rope),
+              lambda: dw.run(q, pool, append_key=k, append_value=k, rope=(0.0, 1e4)),
+              lambda: pw.run(q, pool, sm_scale=-1.0)]
+    hnd = dict(kv_layout="HND")
+    for x in bad_rows:
+        calls += [lambda x=x: pagedattn.append_paged_kv_cache(x, k, *meta_args, **hnd),
+                  lambda x=x: pagedattn.append_paged_kv_cache(k, x, *meta_args, **hnd),
+                  lambda x=x: pagedattn.rope_append_paged_kv_cache(q, x, k, *meta_args, **hnd),
+                  lambda x=x: pagedattn.append_paged_kv_cache_e4m3_amax(
+                      x if x.dtype != torch.float16 else x[:1], k, bi, pos, pool8, ind, indptr,
+                      last, scales)]
+    for x in (bi[:1], torch.cat([bi, bi])):
+        calls += [lambda x=x: pagedattn.append_paged_kv_cache(k, k, x, *meta_args[1:], **hnd),
+                  lambda x=x: pagedattn.rope_append_paged_kv_cache(q, k, k, bi, x, *meta_args[2:],
+                                                                   **hnd)]
+    for x in bad_scales:
+        calls += [lambda x=x: pagedattn.append_paged_kv_cache(k, k, bi, pos, pool8, ind, indptr,
+                                                              last, kv_scales=x, **hnd)]
+    flag = torch.zeros(1, dtype=torch.int32, **dev)
+    calls += [lambda f=f: pagedattn.append_paged_kv_cache(k, k, bi, pos, pool8, ind, indptr, last,
+                                                          kv_scales=scales, error_flag=f, **hnd)
+              for f in (flag, flag.long(), flag.cpu())]
+
+    def errors():
+        got = []
+        for i, call in enumerate(calls):
+            with pytest.raises((ValueError, NotImplementedError, RuntimeError, TypeError)) as e:
+                call()
+                pytest.fail(f"call {i} was taken")
+            got.append((type(e.value), str(e.value)))
+        return got
+
+    with_native = errors()
+    monkeypatch.setattr(pagedattn.ops, "_native", lambda *a: NotImplemented)
+    assert errors() == with_native
