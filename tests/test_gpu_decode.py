@@ -493,15 +493,14 @@ def test_decode_fused_append_counts(gpu):
         assert ws[:8].view(torch.int32).tolist() == [skipped, clamped], split
 
 
-@pytest.mark.parametrize("d,fp8", [(64, False), (128, False), (128, True)])
+@pytest.mark.parametrize("d,fp8,where", [(d, False, w) for d in (64, 128)
+                                         for w in ("q_nan", "k_nan", "v_nan")]
+                         + [(128, True, "q_nan")])
 @pytest.mark.parametrize("split_pages", [8, 64])
-@pytest.mark.parametrize("where", ["q_nan", "k_nan", "v_nan"])
 def test_decode_merge_not_finite(gpu, d, fp8, split_pages, where):
     # a value that is not finite reaches the same outputs and lse whether the
     # sequence is cut or not, up to 8 pieces a row (64-page chunks) and past
     # it: in every piece (a q row) or in one (a K or V row)
-    if fp8 and where != "q_nan":
-        pytest.skip("the pool's rows are finite codes")
     hq, hkv = 8, 2
     meta, pool, q = decode_case(gpu, [3000, 700, 3000], hq, hkv, d, seed=d)
     if where == "q_nan":

@@ -21,7 +21,7 @@ HQ, HKV, D = 16, 2, 128
 @pytest.fixture(autouse=True)
 def _default_planner(monkeypatch):
     for var in ("PAGEDATTN_PREFILL_SPLIT", "PAGEDATTN_DECODE_SHARED",
-                "PAGEDATTN_DECODE_SHARED_SLACK_KB"):
+                "PAGEDATTN_DECODE_SHARED_SLACK_KB", "PAGEDATTN_DECODE_DETERMINISTIC"):
         monkeypatch.delenv(var, raising=False)
 
 
