@@ -1334,14 +1334,29 @@ constexpr int kMergeClasses = 8;
 constexpr int kMergeBatch = 8;
 constexpr int kMergeLoads = 16;
 static_assert(kMergeClasses * kMergeBatch == kWave, "one piece's lse per lane");
-// So eight waves merge a launch of at most 16 rows per piece of its longest row:
-// one sequence of 32000 tokens among 15 of 1000 (512 rows, 87 pieces) runs 42.3 us
-// with eight waves and 47.4 us with D threads, 24 equal ones of 2730 (768 rows,
-// 10 pieces) 53.0 and 51.6 us.  Device partitions do not know their pieces: 256
-// rows, one per CU (8 sequences of 4000 tokens 14.8 against 15.9 us, of 500 12.5
-// against 12.2 us).
-constexpr int kMergeRowsPerPiece = 16;
+// So eight waves (decode_merge_eight) take a host plan of 9 pieces or more on up to
+// 512 rows, two per CU (16 sequences of 4000 tokens equal;
+// 24 of 2730, 768 rows: 53.0 us against 51.6 us), and beyond that a batch with one
+// sequence far longer than the others, whose many pieces the D threads would walk
+// while the others wait: more than 16 pieces, twice the mean of the merged
+// sequences or more, up to 128 rows a piece.  TinyLlama heads, 99 sequences of
+// 700 tokens and one of 40000 (3200 rows): 29.7 us against 32.6 us; 8 KV heads, 64
+// query heads, 32 of 1000 and one of 60000 (2112 rows): 70.8 against 73.4 us; 16
+// sequences of 32 pieces each (2048 rows): 1.5 us the other way.  Device partitions
+// do not know their pieces: 256 rows, one per CU (8 sequences of 4000 tokens 14.8
+// against 15.9 us, of 500 12.5 against 12.2 us).
+constexpr int kMergeRows = 512;
+constexpr int kMergeLong = 16;
+constexpr int kMergeRowsPerPiece = 128;
 constexpr int kMergeDeviceRows = 256;
+
+inline bool decode_merge_eight(int n_merge, int g, int n_slots, int max_pieces) {
+  const int64_t rows = (int64_t)n_merge * g;
+  if (max_pieces <= kMergeClasses) return false;
+  if (rows <= kMergeRows) return true;
+  return max_pieces > kMergeLong && (int64_t)max_pieces * n_merge >= 2 * (int64_t)n_slots &&
+         rows <= (int64_t)kMergeRowsPerPiece * max_pieces;
+}
 
 __device__ __forceinline__ float merge_lane(float v, int i) {
   return __builtin_bit_cast(float,
@@ -1773,9 +1788,7 @@ static int decode_run_impl(const char* who, const pagedattn_plan* plan,
   }
   if (plan->n_merge == 0) return rc;
   const dim3 grid(plan->n_merge, p.g);
-  const bool eight =
-      plan->max_pieces > kMergeClasses &&
-      (int64_t)plan->n_merge * p.g <= (int64_t)kMergeRowsPerPiece * plan->max_pieces;
+  const bool eight = decode_merge_eight(plan->n_merge, p.g, plan->n_slots, plan->max_pieces);
   auto* mfn = plan->d == 64
                   ? (bf16 ? pick_merge<true, 64>(eight) : pick_merge<false, 64>(eight))
                   : (bf16 ? pick_merge<true, 128>(eight) : pick_merge<false, 128>(eight));

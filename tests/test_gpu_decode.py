@@ -70,11 +70,14 @@ def test_decode_balanced_item_cost(gpu, monkeypatch, cost):
 
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("pieces", [[8, 3, 1], [9, 8, 2], [16, 17], [63, 65, 1],
-                                    [17, 16] + [9] * 19, [66, 65] + [2] * 70])
+                                    [17, 16] + [9] * 19, [66, 65] + [2] * 70,
+                                    [9, 10] * 17, [17, 16, 9] * 11, [66] + [40] * 32])
 def test_decode_merge_piece_counts(gpu, d, pieces):
     # fixed chunks of 128 tokens: up to 8 pieces a row (one round trip of the
-    # merge), one past it, and around its 64 pieces per round trip; in the last
-    # two, rows enough for D threads a row (16 and 64 pieces per round trip)
+    # merge), one past it, and around its 64 pieces per round trip.  Sixteen rows
+    # a sequence: up to 512 rows of 9 pieces or more, and the 72 sequences of which
+    # two are long, take eight waves a row, the last three D threads (16 and 64
+    # pieces per round trip)
     lens = [128 * n - (5 if n > 1 else 100) for n in pieces]
     meta, pool, q = decode_case(gpu, lens, 16, 2, d, seed=sum(pieces))
     ref_o, ref_l = oracle_decode(meta, pool, q)
