@@ -118,9 +118,9 @@ __global__ void __launch_bounds__(256) append_kernel(AppendArgs a) {
 // single one up to head_dim 128).  A token's units are its hq q heads, hkv k
 // heads and hkv v heads; 8 lanes (fewer where the head has fewer chunk pairs)
 // work a unit, lane c the 16-byte chunk c of the head's first half and its
-// partner half a head away.  Wave w evaluates token w's cosines and sines, one
-// frequency per lane, into LDS, and the last wave looks the tokens' pages up,
-// while every thread's first rows are already on their way.
+// partner half a head away.  Wave w evaluates the cosines and sines of tokens
+// w, w + 4, ..., one frequency per lane, into LDS, and the last wave looks the
+// tokens' pages up, while every thread's first rows are already on their way.
 //
 // Before, one thread owned (token, 8 frequencies) and walked all heads one
 // after the other: a 512-token step of a 32/8-head layer kept 16 of 256 CUs
@@ -136,8 +136,18 @@ struct RopeAppendArgs {
 };
 
 constexpr int kRopeFreqs = 64;
-constexpr int kRopeMaxTokens = 4;  // one wave's table each
-constexpr int kRopeBatch = 4;      // units a thread has in flight
+constexpr int kRopeMaxTokens = 16;
+constexpr int kRopeWaveTokens = 4;  // up to one table a wave
+constexpr int kRopeBatch = 4;       // units a thread has in flight
+// Layers of few heads take more tokens per workgroup where that leaves 1024
+// workgroups, four per CU: a workgroup of four tokens has little to hide its
+// prologue (tables, page lookups) behind.  8 + 1 heads, D = 128 (80 lanes a token):
+// 4 / 8 / 16 tokens take 8.0 / 8.2 / 9.7 us for 4096 tokens, 11.8 / 10.8 / 11.9 us
+// for 8192, 21.5 / 19.2 / 18.0 us for 16384 and 67.4 / 60.7 / 57.6 us for 65536;
+// 4 + 1 heads, D = 64, 65536 tokens 37.1 / 26.1 / 24.2 us.  The line: at 96 lanes
+// still 85.3 / 80.5 / 80.4 us, at 128 (12 + 2 heads) 100.4 / 100.0 / 102.4 us.
+constexpr int kRopeFewLanes = 96;
+constexpr int kRopeGroups = 1024;
 
 template <bool IS_BF16, bool TO_FP8>
 __global__ void __launch_bounds__(256) rope_append_kernel(RopeAppendArgs r) {
@@ -185,11 +195,13 @@ __global__ void __launch_bounds__(256) rope_append_kernel(RopeAppendArgs r) {
   };
   int u0 = threadIdx.x >> r.c_shift;
   load(u0);
-  if (wave < nt && lane < 8 * npair) {
-    float cs, sn;
-    rope_cos_sin(a.positions[j0 + wave], f0 + lane, d, r.inv_scale, r.log2_theta, &cs, &sn);
-    tab[wave][0][lane] = cs;
-    tab[wave][1][lane] = sn;
+  if (lane < 8 * npair) {
+    for (int t = wave; t < nt; t += 256 / kWave) {
+      float cs, sn;
+      rope_cos_sin(a.positions[j0 + t], f0 + lane, d, r.inv_scale, r.log2_theta, &cs, &sn);
+      tab[t][0][lane] = cs;
+      tab[t][1][lane] = sn;
+    }
   }
   if (wave == 256 / kWave - 1 && lane < nt) {
     int slot = 0;
@@ -533,10 +545,12 @@ int pagedattn_rope_append_paged_kv_cache(
   r.c_shift = 0;
   while ((1 << r.c_shift) < pairs) ++r.c_shift;
   // tokens per workgroup: as many as one batch of loads covers (a token of few
-  // heads does not fill 256 threads by itself)
+  // heads does not fill 256 threads by itself), more for many tokens of few heads
   const int64_t lanes = ((int64_t)num_qo_heads + 2 * (int64_t)num_kv_heads) << r.c_shift;
-  r.tokens = (int)std::min<int64_t>(kRopeMaxTokens,
+  r.tokens = (int)std::min<int64_t>(kRopeWaveTokens,
                                     std::max<int64_t>(1, 256 * kRopeBatch / 2 / lanes));
+  if (lanes <= kRopeFewLanes)
+    r.tokens = std::max(r.tokens, std::min(kRopeMaxTokens, nnz / kRopeGroups));
   const dim3 grid((unsigned)(((int64_t)nnz + r.tokens - 1) / r.tokens),
                   (unsigned)((head_dim / 2 + kRopeFreqs - 1) / kRopeFreqs));
   hipStream_t s = (hipStream_t)stream;

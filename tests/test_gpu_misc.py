@@ -257,6 +257,9 @@ def test_rope_append_equals_separate(gpu, dtype, prefill, fp8):
     (128, 64, 8, 18),   # more units than one batch of loads
     (160, 2, 2, 9),     # two frequency blocks, the second partial
     (256, 16, 16, 3),
+    (48, 1, 1, 17001),  # few heads, many tokens: 16 tokens a workgroup, the last one's partial
+    (64, 4, 1, 5131),   # 5 tokens a workgroup, more than its waves
+    (128, 4, 4, 8197),  # 8 tokens a workgroup, the most lanes a token for that
 ])
 def test_rope_append_shapes_equal_separate(gpu, d, hq, hkv, nnz):
     # the workgroup split of the fused launch at its edges: same bits as the
